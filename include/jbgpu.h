@@ -311,7 +311,9 @@ int jbgpu_solver_set_colouring(jbgpu_ctx* ctx, int32_t degree_first, int32_t rec
 /* ContactSolverInfo.warmstartingFactor for the following solves (0.85 by default). */
 int jbgpu_solver_set_warmstart_factor(jbgpu_ctx* ctx, float factor);
 /* Launch shaping of the colour sweeps (no reference counterpart; results are identical for every
- * value): trailing colours of at most `threshold` manifolds are swept by one single-workgroup launch,
+ * value) where a solve launches them colour by colour (a body with more than 64 colours' manifolds, a body
+ * flagged static that has a mass, or with blocks; every other solve runs all its sweeps in one launch):
+ * trailing colours of at most `threshold` manifolds are swept by one single-workgroup launch,
  * colour after colour; 0 gives every colour its own launch.  Default 1024. */
 int jbgpu_solver_set_tail(jbgpu_ctx* ctx, int32_t threshold);
 /* Residual after each iteration of the last solve (in fixed-iteration mode only the last one). */
@@ -363,13 +365,14 @@ int jbgpu_timing_enable(jbgpu_ctx* ctx, int32_t on);
 int jbgpu_timing_get(jbgpu_ctx* ctx, double* ms, int64_t* launches, int64_t* steps);
 /* Kernel-level timing of the solver sweeps (independent of jbgpu_timing_enable): on every `every`-th
  * solve after this call (0 = off) each sweep launch of every `stride`-th iteration (jbgpu_timing_kernels_stride,
- * default 5) carries its own start/stop events (hipExtLaunchKernel), so the figures are kernel execution time
+ * default 5; a solve whose sweeps run in one launch gives the normal and the friction sweep of a timed iteration a
+ * launch each, and every other iteration one) carries its own start/stop events (hipExtLaunchKernel), so the figures are kernel execution time
  * without launch gaps: summed ms, timed launches and rows processed by them.  Every iteration sweeps the same
  * colours; the events cost about 10 us per launch, which a sampled solve pays. */
 int jbgpu_timing_kernels(jbgpu_ctx* ctx, int32_t every);
 /* The iteration stride of that timing (at least 1; 1 = every iteration). */
 int jbgpu_timing_kernels_stride(jbgpu_ctx* ctx, int32_t stride);
-/* four entries each: [0] normal rows, per-colour launches, [1] friction rows, per-colour launches,
+/* four entries each: [0] normal rows, per-colour or whole-sweep launches, [1] friction rows, the same,
  * [2] normal rows, block launches, [3] friction rows, block launches */
 /* Device memory for callers that keep their own inputs resident in HBM (e.g. AABBs for
  * jbgpu_bp_set_aabbs with on_device = 1) without linking another GPU runtime; freed by the caller. */

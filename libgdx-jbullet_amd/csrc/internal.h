@@ -319,7 +319,7 @@ struct Ctx {
   HBuf<double> solveRh;               // per-iteration (change, norm) sums
   HBuf<unsigned long long> solveRows; // rows in total, rows of the per-colour or block sweeps
   struct {
-    bool pending = false, tolMode = false, blockSweeps = false, sampleK = false;
+    bool pending = false, tolMode = false, blockSweeps = false, sampleK = false, flow = false;
     int iters = 0, sampledIters = 0;  // sampledIters: iterations whose sweep launches were event-timed
     size_t kUsed = 0;
   } solveStat;
@@ -336,6 +336,13 @@ struct Ctx {
   DBuf<int4> hdr;            // per colour slot: point mask | first row << 4, body A, body B, pair index
   DBuf<int> slotCount, slotStart;  // rows per slot and their exclusive prefix sum
   DBuf<float> nrow, frow;    // dense rows: normal row r, friction rows 2r and 2r+1
+  // sweeps in one launch: per slot (rank and degree of body A, of body B, inverse masses); tagged impulses of the
+  // normal and friction rows and tagged body velocities (4 words per body); tickets and error word
+  DBuf<int4> flowDep;
+  DBuf<unsigned long long> flowNapp, flowFapp, flowBody;
+  DBuf<int> flowCtl;
+  HBuf<int> flowErrHost;
+  bool oddBodies = false;  // a body flagged static has a mass
   DBuf<int2> activeBodies;   // per active manifold: body A, body B
   DBuf<int> colorStart;
   HBuf<int> batchHost;  // readback of the colour batches: count, first slots, boundary flags
@@ -363,7 +370,7 @@ struct Ctx {
   DBuf<uint64_t> colorKey, colorKeyAlt;
   DBuf<int> colorOrder, colorOrderAlt;
   std::vector<int64_t> colorOff;
-  DBuf<int> colorOffDev;     // colour offsets on the device (tail sweeps, the per-body warm start)
+  DBuf<int> colorOffDev;     // colour offsets on the device (tail sweeps of the per-colour launches)
   DBuf<int> warmSlotOf;      // per (colour batch, body): the body's slot in the batch, -1 for none
   // block-partitioned sweeps: dynamic bodies in blocks of blockSize consecutive Morton positions; manifolds
   // inside one block ("interior") are swept by one workgroup per block with the block's velocities in LDS,

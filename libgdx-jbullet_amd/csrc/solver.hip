@@ -8,18 +8,18 @@
 // :61-93).  Instead of the reference's Random(0)-shuffled row order the
 // manifolds that carry rows are coloured (Jones-Plassmann with hashed
 // priorities, smallest free colour per round) so that manifolds of one colour
-// share no dynamic body; one thread handles one manifold's points in order and
-// a colour is one launch.  Processing colour after colour is exactly the
+// share no dynamic body.  All sweeps of a solve run in one launch in which a
+// manifold waits for its own two bodies only (kFlowSweep); where that does not
+// apply, a colour is one launch.  Processing colour after colour is exactly the
 // sequential solver fed the manifold order "colour 0 manifolds, colour 1
 // manifolds, ..." (any order inside a colour gives the same bits); the library
 // reports that order so the CPU oracle can be fed the same order.
 //
 // Row storage is in colour-slot order (slot p = position in the colour order):
 // a 16-byte header {point mask, body A, body B, pair index} and the rows of the
-// slot's four contacts, so a sweep thread issues its header and row loads in one
-// round trip and the two body velocities in a second.  Setup is split into a
-// fully parallel row build (rows depend only on the pre-solve state) and a
-// per-colour warm-start application (impulses are applied in manifold order).
+// slot's contacts.  Setup is split into a fully parallel row build (rows depend
+// only on the pre-solve state) and a warm-start application per body (impulses
+// are applied in manifold order).
 #include <cmath>
 
 
@@ -532,7 +532,7 @@ __global__ void kWarmSlotTable(int na, int nBatches, const int* __restrict__ col
                                const float* __restrict__ svel, int nb, int* slotOf) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= na) return;
-  int lo = 0, hi = nBatches;  // the batch of slot p: colorOff[lo] <= p < colorOff[lo + 1]
+  int lo = 0, hi = nBatches;  // the batch of slot p, the last with colorOff[lo] <= p (colorOff: first slots)
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (colorOff[mid] <= p) lo = mid; else hi = mid;
@@ -958,6 +958,384 @@ __global__ __launch_bounds__(kTailThreads) void kFrictionTail(int c0, int c1, co
         frictionQuad(p, threadIdx.x & 3, SP, hdr, nrow, frow, GlobalBodies{svel, props}, dd, nn);
       __syncthreads();
     }
+  accumulate(dd, nn, res);
+}
+
+// ---- every sweep of a solve in one launch ----------------------------------------------------------------
+// A slot of a sweep depends only on the slots that touched its two bodies before it, not on its whole colour: a
+// launch per colour and sweep costs 5-7 us where the dependent arithmetic of one slot takes a fraction of one.
+// Here one launch runs all sweeps of a solve.  Every value a sweep hands on is in 64-bit words that carry a tag
+// (which version it is), written and read with relaxed agent-scope atomics, so a word is never seen half written and
+// no fence or flag is needed: four words per body (48 bits of velocity and a 16-bit tag each; the tag counts the
+// updates the body has had, modulo 2^16) and one word per row for its applied impulse {float bits, iterations}.
+// Slot p of sweep w (normal and friction sweeps alternate) waits until body X carries tag w * deg(X) + rank(X, p),
+// deg(X) the body's slots and rank the position of p among them in colour order, and leaves tag + 1: each body sees
+// exactly the sequence of the colour-by-colour sweeps.  A body has at most one slot per colour, so rank and degree
+// are bit counts in its colour mask (colours below 64).  Bodies that are static carry no tag and are read from svel.
+// A body cannot move past the version a slot waits for, so a word found ready is not read again, and a 16-bit tag
+// cannot be mistaken for one 2^16 updates away.
+//
+// Progress: the groups of a sweep (16 slots of one colour, four lanes each) are numbered in sweep and colour order,
+// and a workgroup (one wave) takes group after group by tickets in that order; a group only waits for groups before
+// it, which are finished or held by running waves, so the smallest unfinished group can always go on, whatever part
+// of the grid is resident.  Tickets are dealt in kFlowShards interleaved sequences (same-address atomics take about
+// 11 ns each); a workgroup's sequence is its starting order modulo kFlowShards, so each sequence has a running
+// workgroup once kFlowShards have started, and a workgroup leaves only when its sequence is used up.  Waits are
+// bounded all the same and raise an error word.
+//
+// Within a group, each slot runs once its own two bodies are ready (a hub body's next slot does not wait for the
+// group's slowest); a wave whose slots are all more than one update away sleeps between polls.
+typedef unsigned long long flow_t;
+constexpr int kFlowShards = 16;
+// control words (ints, 128 bytes apart): starting order, one ticket counter per sequence, error (sticky)
+constexpr int kFlowCtlTicket = 32, kFlowCtlStride = 32;
+constexpr int kFlowCtlErr = kFlowCtlTicket + kFlowCtlStride * kFlowShards;
+constexpr int kFlowCtlWords = kFlowCtlErr + kFlowCtlStride;
+constexpr int kFlowMaxColours = 64;
+constexpr int kFlowSlots = 16;           // slots per group (one wave, four lanes per slot)
+constexpr int kFlowSpinLimit = 1 << 22;  // polls of one group (about a microsecond each)
+
+__device__ __forceinline__ flow_t flowLoad(const flow_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void flowStore(flow_t* p, flow_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// impulse words
+__device__ __forceinline__ flow_t flowImpulse(float v, int tag) {
+  return ((flow_t)(unsigned)tag << 32) | __float_as_uint(v);
+}
+__device__ __forceinline__ float flowValue(flow_t w) { return __uint_as_float((unsigned)w); }
+__device__ __forceinline__ int flowTag(flow_t w) { return (int)(unsigned)(w >> 32); }
+// velocity words: a vector's 96 bits in the low 48 bits of two words, the tag above
+__device__ __forceinline__ void flowPack(V3 v, unsigned tag, flow_t& w0, flow_t& w1) {
+  const unsigned y = __float_as_uint(v.y);
+  w0 = ((flow_t)((tag << 16) | (y & 0xffffu)) << 32) | __float_as_uint(v.x);
+  w1 = ((flow_t)((tag << 16) | (y >> 16)) << 32) | __float_as_uint(v.z);
+}
+__device__ __forceinline__ V3 flowUnpack(flow_t w0, flow_t w1) {
+  const unsigned y = ((unsigned)(w0 >> 32) & 0xffffu) | ((unsigned)(w1 >> 32) << 16);
+  return v3(__uint_as_float((unsigned)w0), __uint_as_float(y), __uint_as_float((unsigned)w1));
+}
+__device__ __forceinline__ unsigned flowVersion(flow_t w) { return (unsigned)(w >> 48); }
+
+// tagged words of a solve from its rows and solver bodies (all tags 0); per slot (rank and degree of body A, of body
+// B, inverse masses); four lanes per slot
+__global__ void kFlowInit(int na, int nb, const int4* __restrict__ hdr, const int* __restrict__ corder,
+                          const int* __restrict__ color, const unsigned long long* __restrict__ bodyMask,
+                          const float* __restrict__ props, const float* __restrict__ svel,
+                          const float* __restrict__ nrow, const float* __restrict__ frow, int4* dep, flow_t* napp,
+                          flow_t* fapp, flow_t* body, int* ctl) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < kFlowCtlWords) ctl[t] = 0;
+  if (t < nb) {
+    const float4* s = (const float4*)(svel + 8 * (size_t)t);
+    const float4 a = s[0], b = s[1];
+    flow_t* w = body + 4 * (size_t)t;
+    flowPack(v3(a.x, a.y, a.z), 0, w[0], w[1]);
+    flowPack(v3(b.x, b.y, b.z), 0, w[2], w[3]);
+  }
+  const int p = t >> 2, q = t & 3;
+  if (p >= na) return;
+  const int4 h = hdr[p];
+  const int r = slotRow(h) + q;
+  if (q < __popc(slotMask(h))) {
+    napp[r] = flowImpulse(nrow[(size_t)RW * r + 19], 0);
+    fapp[2 * (size_t)r] = flowImpulse(frow[(size_t)RW * (2 * r) + 19], 0);
+    fapp[2 * (size_t)r + 1] = flowImpulse(frow[(size_t)RW * (2 * r + 1) + 19], 0);
+  }
+  if (q) return;
+  const unsigned long long below = (1ull << color[corder[p]]) - 1;
+  int4 d = make_int4(0, 0, __float_as_int(svel[8 * (size_t)h.y + 3]), __float_as_int(svel[8 * (size_t)h.z + 3]));
+  if (dynamicBody(props, h.y)) d.x = __popcll(bodyMask[h.y] & below) | (__popcll(bodyMask[h.y]) << 16);
+  if (dynamicBody(props, h.z)) d.y = __popcll(bodyMask[h.z] & below) | (__popcll(bodyMask[h.z]) << 16);
+  dep[p] = d;
+}
+
+// what every group of a launch reads and writes
+struct FlowSweep {
+  const int4* __restrict__ hdr;
+  const int4* __restrict__ dep;
+  float* nrow;
+  float* frow;
+  flow_t* napp;
+  flow_t* fapp;
+  flow_t* body;
+  float* svel;
+  int* ctl;
+};
+// the group a wave works on: the quad's slot (none: valid false) in sweep `sweep` of the launch
+struct FlowGroup {
+  int4 h, d;
+  bool valid;
+  int sweep;
+};
+
+// One row on a quad: lane q holds one of the four vectors a row touches, linear (q even) or angular (q odd) velocity
+// of body A (q < 2) or B, in v, the row's part that multiplies it (D) and the change of it per unit impulse (U).  The
+// four products meet by DPP; the scalars of row L sit in lane L.  A row costs its dot product, two DPP steps and one
+// update per lane, about 30 instructions, where one lane doing a whole row (and handing both bodies on to the next
+// point's lane) took about 70: on the critical path of a body with many slots that is time per update.
+__device__ __forceinline__ float quadPairSum(float x) {  // x of this lane and of its neighbour (lanes 0/1, 2/3)
+  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float flowRelVel(V3 D, V3 v) {  // (nrm.A.lv + r1.A.av) - (nrm.B.lv + r2.B.av)
+  const float s = quadPairSum(dot(D, v));
+  return quadBcast<0>(s) - quadBcast<2>(s);
+}
+__device__ __forceinline__ void flowApply(V3& v, V3 U, float imp, int q, bool moves) {
+  const float m = q < 2 ? imp : -imp;
+  if (moves) {
+    v.x += m * U.x;
+    v.y += m * U.y;
+    v.z += m * U.z;
+  }
+}
+// normal row of point L: resolveSingleCollisionCombinedCacheFriendly (:234-284)
+template <int L>
+__device__ __forceinline__ void flowNormalRound(int q, int nr, bool moves, const V3* D, const V3* U, float pimp,
+                                                float rest, float jac, float old, V3& v, float& out) {
+  if (!__any(nr > L)) return;
+  if (nr > L) {
+    const float velocityError = quadBcast<L>(rest) - flowRelVel(D[L], v);
+    const float vimp = velocityError * quadBcast<L>(jac);
+    float ni = quadBcast<L>(pimp) + vimp;
+    const float was = quadBcast<L>(old);
+    const float sum = was + ni;
+    const float nw = 0.0f > sum ? 0.0f : sum;
+    ni = nw - was;
+    flowApply(v, U[L], ni, q, moves);
+    if (q == L) out = nw;
+  }
+}
+// one friction row of point L: resolveSingleFrictionCacheFriendly (:286-346)
+template <int L>
+__device__ __forceinline__ void flowFrictionRow(int q, bool moves, V3 D, V3 U, float total, float fric, float jac,
+                                                float old, V3& v, float& out) {
+  const float limit = quadBcast<L>(total) * quadBcast<L>(fric);
+  const float j1 = -flowRelVel(D, v) * quadBcast<L>(jac);
+  const float was = quadBcast<L>(old);
+  float ap = was + j1;
+  if (limit < ap) {
+    ap = limit;
+  } else if (ap < -limit) {
+    ap = -limit;
+  }
+  flowApply(v, U, ap - was, q, moves);
+  if (q == L) out = ap;
+}
+template <int L>
+__device__ __forceinline__ void flowFrictionRound(int q, int nr, bool moves, const V3* D, const V3* U, float total,
+                                                  float fric0, float jac0, float old0, float fric1, float jac1,
+                                                  float old1, V3& v, float& out0, float& out1) {
+  if (!__any(nr > L)) return;
+  if (nr > L && quadBcast<L>(total) > 0.0f) {
+    flowFrictionRow<L>(q, moves, D[2 * L], U[2 * L], total, fric0, jac0, old0, v, out0);
+    flowFrictionRow<L>(q, moves, D[2 * L + 1], U[2 * L + 1], total, fric1, jac1, old1, v, out1);
+  }
+}
+
+// one group in iteration `it`, normal or friction rows.  Returns false when the wait gave up.
+template <bool Fr>
+__device__ __forceinline__ bool flowRun(const FlowSweep& W, const SolverParams& SP, const FlowGroup& G, int it,
+                                        bool track, bool last, double& dd, double& nn) {
+  const int lane = threadIdx.x & 63, q = lane & 3;
+  const int4 h = G.h, d = G.d;
+  const int nr = __popc(slotMask(h));
+  const bool mine = q < nr;  // lane q keeps the scalars and impulses of the slot's q-th point
+  const int row0 = slotRow(h), r = row0 + q;
+  const int x = q < 2 ? h.y : h.z;  // this lane's body
+  const int rd = q < 2 ? d.x : d.y;
+  const float invMass = __int_as_float(q < 2 ? d.z : d.w);
+  const int deg = rd >> 16, rank = rd & 0xffff;
+  const unsigned want = ((unsigned)(2 * it + (Fr ? 1 : 0)) * (unsigned)deg + (unsigned)rank) & 0xffffu;
+  flow_t* bw = W.body + 4 * (size_t)x + 2 * (q & 1);
+  // rows: normal(3) rel1xn(3) rel2xn(3) angA(3) angB(3) jacInv pen rest fric applied
+  constexpr int NV = Fr ? 8 : 4;  // rows of the slot
+  V3 D[NV], U[NV];
+  float s15 = 0.0f, s16 = 0.0f, s17 = 0.0f, s18 = 0.0f;  // normal: jacInv, pen, rest; friction: jacInv and fric of both
+  {
+    const int od = q == 1 ? 3 : q == 3 ? 6 : 0, ou = q == 1 ? 9 : q == 3 ? 12 : 0;
+    const float scale = q & 1 ? 1.0f : invMass;  // linear: the normal times the inverse mass
+    const float* rows = (Fr ? W.frow + (size_t)RW * (2 * row0) : W.nrow + (size_t)RW * row0);
+    if (mine) {
+      const float* S = rows + (size_t)RW * (Fr ? 2 * q : q);
+      s15 = S[15];
+      if (Fr) {
+        s16 = S[18];
+        s17 = S[RW + 15];
+        s18 = S[RW + 18];
+      } else {
+        s16 = S[16];
+        s17 = S[17];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+      D[j] = U[j] = v3(0.0f, 0.0f, 0.0f);
+      if ((Fr ? j >> 1 : j) < nr) {
+        D[j] = ld3(rows + RW * j + od);
+        U[j] = scl(ld3(rows + RW * j + ou), scale);
+      }
+    }
+  }
+  const bool dyn = deg > 0, moves = invMass != 0.0f;
+  V3 v = v3(0.0f, 0.0f, 0.0f);
+  if (G.valid && !dyn) v = ld3(W.svel + 8 * (size_t)x + 4 * (q & 1));  // a static body's constant velocity
+  // two static bodies (a caller's island list): nothing orders the sweeps of this slot but its own impulses
+  const bool fixed = (d.x | d.y) == 0;
+  float old0 = 0.0f, old1 = 0.0f, total = 0.0f, pimp = 0.0f;
+  bool pending = G.valid, needBody = G.valid && dyn, needImp = mine;
+  for (int spin = 0;; spin++) {
+    int away = 0;  // updates this lane's body still has to see
+    flow_t w0 = 0, w1 = 0, n0 = 0, f0 = 0, f1 = 0;
+    if (needBody) {
+      w0 = flowLoad(bw);
+      w1 = flowLoad(bw + 1);
+    }
+    if (needImp) {
+      n0 = flowLoad(W.napp + r);
+      if (Fr || fixed) {
+        f0 = flowLoad(W.fapp + 2 * (size_t)r);
+        f1 = flowLoad(W.fapp + 2 * (size_t)r + 1);
+      }
+    }
+    if (!Fr && spin == 0) {  // the part of the impulse without velocities, while the first polls are out
+      const float positionalError = -s16 * SP.erp / SP.dt;
+      pimp = positionalError * s15;
+    }
+    if (needBody) {
+      needBody = flowVersion(w0) != want || flowVersion(w1) != want;
+      away = (int)((want - flowVersion(w0)) & 0xffffu);
+      v = flowUnpack(w0, w1);
+    }
+    if (needImp) {
+      needImp = flowTag(n0) != it + (Fr ? 1 : 0);
+      if (Fr || fixed) needImp = needImp || flowTag(f0) != it || flowTag(f1) != it;
+      if (Fr) {
+        total = flowValue(n0) + 0.0f;  // appliedImpulse + appliedPushImpulse (0)
+        old0 = flowValue(f0);
+        old1 = flowValue(f1);
+      } else {
+        old0 = flowValue(n0);
+      }
+    }
+    const unsigned long long waiting = __ballot(needBody || needImp);
+    const bool go = pending && ((waiting >> (lane & ~3)) & 15) == 0;
+    if (go) {
+      float out0 = old0, out1 = old1;
+      if (Fr) {
+        flowFrictionRound<0>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
+        flowFrictionRound<1>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
+        flowFrictionRound<2>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
+        flowFrictionRound<3>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
+      } else {
+        flowNormalRound<0>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
+        flowNormalRound<1>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
+        flowNormalRound<2>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
+        flowNormalRound<3>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
+      }
+      if (dyn) {
+        flow_t o0, o1;
+        flowPack(v, (want + 1) & 0xffffu, o0, o1);
+        flowStore(bw, o0);
+        flowStore(bw + 1, o1);
+      }
+      if (mine) {
+        if (Fr) {
+          flowStore(W.fapp + 2 * (size_t)r, flowImpulse(out0, it + 1));
+          flowStore(W.fapp + 2 * (size_t)r + 1, flowImpulse(out1, it + 1));
+        } else {
+          flowStore(W.napp + r, flowImpulse(out0, it + 1));
+        }
+        if (track) {
+          double e = (double)out0 - (double)old0;
+          dd += e * e;
+          nn += (double)out0 * (double)out0;
+          if (Fr) {
+            e = (double)out1 - (double)old1;
+            dd += e * e;
+            nn += (double)out1 * (double)out1;
+          }
+        }
+        if (last) {  // the solve's results, for the kernels after this launch
+          if (Fr) {
+            W.frow[(size_t)RW * (2 * r) + 19] = out0;
+            W.frow[(size_t)RW * (2 * r + 1) + 19] = out1;
+          } else {
+            W.nrow[(size_t)RW * r + 19] = out0;
+          }
+        }
+      }
+      if (Fr && last && dyn && rank == deg - 1) st3(W.svel + 8 * (size_t)x + 4 * (q & 1), v);  // the body's last update
+    }
+    pending = pending && !go;
+    if (!__any(pending)) return true;
+    if (spin >= kFlowSpinLimit) return false;
+    if ((spin & 1023) == 1023 && __hip_atomic_load(W.ctl + kFlowCtlErr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return false;
+    const bool near = ((__ballot(away <= 1) >> (lane & ~3)) & 15) == 15;
+    if (!__any(pending && near)) __builtin_amdgcn_s_sleep(8);
+  }
+}
+
+// sweeps [sweep0, sweep0 + sweeps) of a solve (iteration i: sweeps 2i, normal rows, and 2i + 1, friction rows);
+// starts[k] the first slot of colour k; trackIt: the iteration whose residual terms are accumulated into res (-1: none)
+__global__ __launch_bounds__(64) void kFlowSweep(int na, int ncol, const int* __restrict__ starts, int sweep0,
+                                                 int sweeps, int trackIt, SolverParams SP, FlowSweep W, double* res,
+                                                 const int* __restrict__ done) {
+  if (done && *done) return;  // tolerance mode only
+  const int lane = threadIdx.x;
+  // lane k holds colour k's slots and its first group
+  const int lo = lane < ncol ? starts[lane] : na;
+  const int hi = lane + 1 < ncol ? starts[lane + 1] : na;
+  const int groups = (hi - lo + kFlowSlots - 1) / kFlowSlots;
+  int end = groups;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(end, off);
+    if (lane >= off) end += o;
+  }
+  const int first = end - groups;
+  const int total = __builtin_amdgcn_readlane(end, 63);  // groups per sweep
+  const int limit = total * sweeps;
+  int shard = 0, next = 0;
+  if (lane == 0) shard = atomicAdd(W.ctl, 1) % kFlowShards;
+  shard = __builtin_amdgcn_readfirstlane(shard);
+  int* ticket = W.ctl + kFlowCtlTicket + kFlowCtlStride * shard;
+  if (lane == 0) next = atomicAdd(ticket, 1);
+  // the next group's headers are loaded while the current group waits, and the ticket after it is taken
+  auto fetch = [&](FlowGroup& G) {
+    const int k = __builtin_amdgcn_readfirstlane(next) * kFlowShards + shard;
+    G.sweep = k < limit ? k / total : -1;
+    G.h = make_int4(0, 0, 0, 0);
+    G.d = make_int4(0, 0, 0, 0);
+    G.valid = false;
+    if (G.sweep < 0) return;
+    if (lane == 0) next = atomicAdd(ticket, 1);
+    const int g = k - G.sweep * total;
+    const int c = __popcll(__ballot(lane < ncol && first <= g)) - 1;
+    const int p = __builtin_amdgcn_readlane(lo, c) + (g - __builtin_amdgcn_readlane(first, c)) * kFlowSlots + (lane >> 2);
+    G.valid = p < __builtin_amdgcn_readlane(hi, c);
+    if (G.valid) {
+      G.h = W.hdr[p];
+      G.d = W.dep[p];
+    }
+  };
+  double dd = 0.0, nn = 0.0;
+  FlowGroup G, N;
+  fetch(G);
+  while (G.sweep >= 0) {
+    const int w = sweep0 + G.sweep, it = w >> 1;
+    const bool last = G.sweep + 2 >= sweeps;  // the launch's last normal and friction sweeps
+    fetch(N);
+    const bool ok = w & 1 ? flowRun<true>(W, SP, G, it, it == trackIt, last, dd, nn)
+                                : flowRun<false>(W, SP, G, it, it == trackIt, last, dd, nn);
+    if (!ok) {
+      if (lane == 0) atomicOr(W.ctl + kFlowCtlErr, 1);
+      break;
+    }
+    G = N;
+  }
   accumulate(dd, nn, res);
 }
 
@@ -1759,7 +2137,15 @@ __device__ __forceinline__ void hingeSolve(const float* R, float* S, float dt, S
     applyTorqueImpulse(B, sub(scl(motorImp, -1.0f), angularLimit), IB);
   }
 }
-__device__ void jointSolve(int j, float dt, const float* __restrict__ rec, float* st, float* svel) {
+// flow: the tagged velocity words of the contact sweeps (null: none), whose values follow svel and whose tags stay
+__device__ __forceinline__ void storeBodyFlow(flow_t* flow, int i, const SBody& s) {
+  if (!flow) return;
+  flow_t* w = flow + 4 * (size_t)i;
+  const unsigned tag = flowVersion(w[0]);
+  flowPack(s.lv, tag, w[0], w[1]);
+  flowPack(s.av, tag, w[2], w[3]);
+}
+__device__ void jointSolve(int j, float dt, const float* __restrict__ rec, float* st, float* svel, flow_t* flow) {
   const float* R = rec + kJointWords * j;
   float* S = st + kJointStateWords * j;
   const int a = jointBodyA(R), b = jointBodyB(R);
@@ -1773,16 +2159,23 @@ __device__ void jointSolve(int j, float dt, const float* __restrict__ rec, float
   if (jointType(R) == kJointHinge) hingeSolve(R, S, dt, A, B);
   else p2pSolve(R, S, dt, A, B);
   // a body without inverse mass keeps its record (the reference's read-back skips it as well)
-  if (A.invMass != 0.0f) storeBody(svel, a, A);
-  if (b >= 0 && B.invMass != 0.0f) storeBody(svel, b, B);
+  if (A.invMass != 0.0f) {
+    storeBody(svel, a, A);
+    storeBodyFlow(flow, a, A);
+  }
+  if (b >= 0 && B.invMass != 0.0f) {
+    storeBody(svel, b, B);
+    storeBodyFlow(flow, b, B);
+  }
 }
 // one joint colour per launch: joints [off, off + cnt) of the order
 __global__ void kJointSweep(int off, int cnt, float dt, const int* __restrict__ order, const int* __restrict__ solve,
-                            const float* __restrict__ rec, float* st, float* svel, const int* __restrict__ done) {
+                            const float* __restrict__ rec, float* st, float* svel, flow_t* flow,
+                            const int* __restrict__ done) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= cnt || (done && *done)) return;
   const int j = order[off + k];
-  if (solve[j]) jointSolve(j, dt, rec, st, svel);
+  if (solve[j]) jointSolve(j, dt, rec, st, svel, flow);
 }
 // every joint colour in one workgroup, colour after colour, separated by workgroup barriers
 constexpr int kJointTailThreads = 1024;
@@ -1790,13 +2183,14 @@ __global__ __launch_bounds__(kJointTailThreads) void kJointSweepAll(int ncol, co
                                                                     float dt, const int* __restrict__ order,
                                                                     const int* __restrict__ solve,
                                                                     const float* __restrict__ rec, float* st,
-                                                                    float* svel, const int* __restrict__ done) {
+                                                                    float* svel, flow_t* flow,
+                                                                    const int* __restrict__ done) {
   if (done && *done) return;
   for (int c = 0; c < ncol; c++) {
     const int a = colourOff[c], e = colourOff[c + 1];
     for (int k = a + (int)threadIdx.x; k < e; k += kJointTailThreads) {
       const int j = order[k];
-      if (solve[j]) jointSolve(j, dt, rec, st, svel);
+      if (solve[j]) jointSolve(j, dt, rec, st, svel, flow);
     }
     __syncthreads();
   }
@@ -1901,20 +2295,21 @@ struct JointPass {
       hipLaunchKernelGGL(kJointBuild, dim3(gridFor(c.nj)), dim3(256), 0, c.stream, c.nj, (const float*)c.joints.p,
                          (const int*)c.jointSolve.p, (const float*)c.tr.p, (const float*)c.props.p, c.jointState.p);
   }
-  int sweep(float dt, const int* done) {  // one iteration's constraints; returns the launches
+  int sweep(float dt, const int* done, flow_t* flow = nullptr) {  // one iteration's constraints; returns the launches
     if (!on) return 0;
     const int ncol = (int)c.jointColourOff.size() - 1;
     if (c.nj <= 4 * kJointTailThreads) {
       hipLaunchKernelGGL(kJointSweepAll, dim3(1), dim3(kJointTailThreads), 0, c.stream, ncol,
                          (const int*)c.jointColourOffDev.p, dt, (const int*)c.jointOrder.p,
-                         (const int*)c.jointSolve.p, (const float*)c.joints.p, c.jointState.p, c.svel.p, done);
+                         (const int*)c.jointSolve.p, (const float*)c.joints.p, c.jointState.p, c.svel.p, flow,
+                         done);
       return 1;
     }
     for (int k = 0; k < ncol; k++) {
       const int cnt = c.jointColourOff[k + 1] - c.jointColourOff[k];
       hipLaunchKernelGGL(kJointSweep, dim3(gridFor(cnt)), dim3(256), 0, c.stream, c.jointColourOff[k], cnt, dt,
                          (const int*)c.jointOrder.p, (const int*)c.jointSolve.p, (const float*)c.joints.p,
-                         c.jointState.p, c.svel.p, done);
+                         c.jointState.p, c.svel.p, flow, done);
     }
     return ncol;
   }
@@ -2102,6 +2497,7 @@ void solveWorldBlocks(Ctx& c, float dt, int na, const int* dna = nullptr) {
   c.solveStat.pending = true;
   c.solveStat.tolMode = false;
   c.solveStat.blockSweeps = false;
+  c.solveStat.flow = false;
   c.solveStat.sampleK = false;
   c.solveStat.iters = iters;
   c.solveStat.kUsed = 0;
@@ -2314,6 +2710,7 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   c.batchHost.ensure(2 + 2 * (size_t)kMaxBatches);
   int* hb = c.batchHost.p;
   const unsigned long long* skey = nullptr;  // the sorted slot keys
+  int firstBatches = 0;  // colours before any recolouring pass (colours are contiguous: all below 64 if at most 64)
   auto order = [&]() {
     if (round >= (1 << 10) - 64) throw std::runtime_error("colour index exceeds the slot key");
     hipLaunchKernelGGL(kSlotKeys, dim3(gridFor(na)), dim3(256), 0, s, na, phase, (const int*)c.color.p, c.slotKey.p,
@@ -2348,6 +2745,7 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
       colourPass(rem);
       order();
     }
+    firstBatches = hb[0];
     c.colourRounds = batches <= 1 ? firstRounds - 1 : round;
     for (int pass = 0; pass < c.recolourPasses; pass++) {
       // iterated greedy: the colour classes from the last to the first, every manifold of a class moved to the
@@ -2424,7 +2822,14 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
     if (c.ncolors - headColors < 2) headColors = c.ncolors;
   }
   c.headColors = headColors;
-  if (headColors < c.ncolors) {
+  const bool manyColours = firstBatches > kFlowMaxColours;
+  // All sweeps of an iteration (of the whole solve, where neither constraints nor a residual test stand between
+  // iterations) are one launch; one launch per colour where blocks are swept apart, where a colour lies past the
+  // bodies' 64-bit masks, or where a body flagged static has a mass (its slots share colours).  The 100k pile (243k
+  // slots, 24 colours, 20 iterations): 4.96 ms in 560 launches, 2.48 ms in one; 7.1k slots, 17 colours: 3.04 and
+  // 1.14 ms; 1.3k slots, 7 colours, 10 iterations: 0.55 and 0.23 ms.
+  const bool flow = !blocked && !manyColours && !c.oddBodies;
+  if (!flow && headColors < c.ncolors) {
     std::vector<int> offs(c.colorOff.begin(), c.colorOff.end());
     c.colorOffDev.ensure(offs.size());
     JB_CHECK(hipMemcpyAsync(c.colorOffDev.p, offs.data(), offs.size() * sizeof(int), hipMemcpyHostToDevice, s));
@@ -2440,19 +2845,14 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   int setupLaunches = 1;
   if (apply && !blockSweeps && c.ncolors <= kWarmGatherBatches) {  // warm start gathered per body
     c.warmSlotOf.ensure((size_t)c.ncolors * c.nb);
-    if (c.headColors >= c.ncolors) {  // the batch offsets on the device (already there when a tail is swept)
-      std::vector<int> offs(c.colorOff.begin(), c.colorOff.end());
-      c.colorOffDev.ensure(offs.size());
-      JB_CHECK(hipMemcpyAsync(c.colorOffDev.p, offs.data(), offs.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    }
     JB_CHECK(hipMemsetAsync(c.warmSlotOf.p, 0xff, (size_t)c.ncolors * c.nb * sizeof(int), s));
-    hipLaunchKernelGGL(kWarmSlotTable, dim3(gridFor(na)), dim3(256), 0, s, na, c.ncolors, (const int*)c.colorOffDev.p,
+    hipLaunchKernelGGL(kWarmSlotTable, dim3(gridFor(na)), dim3(256), 0, s, na, c.ncolors, (const int*)c.colorStart.p,
                        (const int4*)c.hdr.p, (const float*)c.svel.p, c.nb, c.warmSlotOf.p);
     hipLaunchKernelGGL(kWarmGather, dim3(gridFor(c.nb)), dim3(256), 0, s, c.nb, c.ncolors,
                        (const int*)c.warmSlotOf.p, (const int4*)c.hdr.p, (const float*)c.nrow.p,
                        (const float*)c.frow.p, (const float*)c.props.p, c.svel.p);
     setupLaunches += 2;
-  } else if (apply) {  // warm start colour by colour: the head colours one launch each, the tail in one workgroup
+  } else if (apply) {  // warm start colour by colour (never with the one-launch sweeps: blocks or over 256 batches)
     for (int k = 0; k < headColors; k++) {
       int cnt = (int)(c.colorOff[k + 1] - c.colorOff[k]);
       hipLaunchKernelGGL(kWarmApply, dim3(gridFor(cnt, 64)), dim3(64), 0, s, (int)c.colorOff[k], cnt, c.hdr.p,
@@ -2525,14 +2925,61 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   int jointLaunches = 0;
   int launchedIters = iters;
   if (tolMode) c.doneHost.ensure(1);
-  for (int itn = 0; itn < iters; itn++) {
+  int64_t flowLaunches = 0;
+  // one launch of `sweeps` sweeps from sweep0 on; timed: with its own events
+  auto flowSweep = [&](int sweep0, int sweeps, double* res, bool timed) {
+    // Waves beyond what the dependences keep busy only poll (their reads go past the L2).  Solve time by grid:
+    // 243k slots (15.2k groups) 2.93 ms at 768 waves, 2.48 at 1536, 2.57 at 2048, 2.93 at 4096; 7.1k slots (460 groups)
+    // 1.20 ms at 128, 1.14 at 192 and 256, 1.19 at 512; 1.3k slots (85 groups) 0.245 ms at 64, 0.225 at 128 to 256.
+    const int groups = na / kFlowSlots + c.ncolors;  // at least the groups of a sweep
+    const int grid = std::min(1536, std::max(128, groups / 2));
+    static_assert(kFlowShards <= 128, "every ticket sequence needs a workgroup");
+    if (sweep0 > 0) JB_CHECK(hipMemsetAsync(c.flowCtl.p, 0, kFlowCtlErr * sizeof(int), s));  // not the error word
+    const FlowSweep W{c.hdr.p, c.flowDep.p, c.nrow.p, c.frow.p, c.flowNapp.p, c.flowFapp.p, c.flowBody.p, c.svel.p,
+                      c.flowCtl.p};
+    const int trackIt = res ? (sweep0 + sweeps - 1) >> 1 : -1;
+    if (timed) {
+      hipEvent_t* ev = kPair(sweep0 & 1);
+      hipExtLaunchKernelGGL(kFlowSweep, dim3(grid), dim3(64), 0, s, ev[0], ev[1], 0, na, c.ncolors,
+                            (const int*)c.colorStart.p, sweep0, sweeps, trackIt, SP, W, res, (const int*)done);
+    } else {
+      hipLaunchKernelGGL(kFlowSweep, dim3(grid), dim3(64), 0, s, na, c.ncolors, (const int*)c.colorStart.p, sweep0,
+                         sweeps, trackIt, SP, W, res, (const int*)done);
+    }
+    flowLaunches++;
+  };
+  if (flow) {
+    c.flowDep.ensure(na);
+    c.flowNapp.ensure(4 * (size_t)na);
+    c.flowFapp.ensure(8 * (size_t)na);
+    c.flowBody.ensure(4 * (size_t)c.nb);
+    c.flowCtl.ensure(kFlowCtlWords);
+    hipLaunchKernelGGL(kFlowInit, dim3(gridFor(std::max<int64_t>({4 * (int64_t)na, c.nb, kFlowCtlWords}))), dim3(256), 0,
+                       s, na, c.nb, (const int4*)c.hdr.p, (const int*)c.colorOrder.p, (const int*)c.color.p,
+                       (const unsigned long long*)c.bodyMask.p, (const float*)c.props.p, (const float*)c.svel.p,
+                       (const float*)c.nrow.p, (const float*)c.frow.p, c.flowDep.p, c.flowNapp.p, c.flowFapp.p,
+                       c.flowBody.p, c.flowCtl.p);
+  }
+  const bool oneLaunch = flow && !tolMode && !jp.on && !sampleK && iters > 0;
+  if (oneLaunch) {
+    double* res = c.resid.p + histWords + 2 * (size_t)kResidStripes * (iters - 1);
+    flowSweep(0, 2 * iters, res, false);
+    hipLaunchKernelGGL(kResidual, dim3(1), dim3(64), 0, s, iters - 1, c.tolerance, res, c.resid.p, c.done.p, resOut);
+  }
+  for (int itn = 0; itn < iters && !oneLaunch; itn++) {
     const bool track = tolMode || itn == iters - 1;
+    double* res = track ? c.resid.p + histWords + 2 * (size_t)kResidStripes * itn : nullptr;
+    jointLaunches += jp.sweep(dt, done, flow ? c.flowBody.p : nullptr);  // the constraints first in every iteration (:823-842)
     sampleIt = sampleK && itn % c.kernelStride == 0;
     sampledIters += sampleIt ? 1 : 0;
-    double* res = track ? c.resid.p + histWords + 2 * (size_t)kResidStripes * itn : nullptr;
-    jointLaunches += jp.sweep(dt, done);  // the constraints first in every iteration (:823-842)
+    if (flow && sampleIt) {  // a timed iteration: its two sweeps apart
+      flowSweep(2 * itn, 1, res, true);
+      flowSweep(2 * itn + 1, 1, res, true);
+    } else if (flow) {
+      flowSweep(2 * itn, 2, res, false);
+    }
     sweepBlocks(false, res);
-    for (int k = firstColor; k < headColors; k++) {
+    for (int k = firstColor; k < headColors && !flow; k++) {
       int cnt = (int)(c.colorOff[k + 1] - c.colorOff[k]);
       if (sampleIt) {
         hipEvent_t* ev = kPair(0);
@@ -2544,12 +2991,12 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
                            c.nrow.p, c.props.p, c.svel.p, res, done);
       }
     }
-    if (headColors < c.ncolors)
+    if (!flow && headColors < c.ncolors)
       hipLaunchKernelGGL(kNormalTail, dim3(1), dim3(kTailThreads), 0, s, headColors, c.ncolors,
                          (const int*)c.colorOffDev.p, SP, (const int4*)c.hdr.p, c.nrow.p, (const float*)c.props.p,
                          c.svel.p, res, (const int*)done);
     sweepBlocks(true, res);
-    for (int k = firstColor; k < headColors; k++) {
+    for (int k = firstColor; k < headColors && !flow; k++) {
       int cnt = (int)(c.colorOff[k + 1] - c.colorOff[k]);
       if (sampleIt) {
         hipEvent_t* ev = kPair(1);
@@ -2561,7 +3008,7 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
                            c.hdr.p, c.nrow.p, c.frow.p, c.props.p, c.svel.p, res, done);
       }
     }
-    if (headColors < c.ncolors)
+    if (!flow && headColors < c.ncolors)
       hipLaunchKernelGGL(kFrictionTail, dim3(1), dim3(kTailThreads), 0, s, headColors, c.ncolors,
                          (const int*)c.colorOffDev.p, SP, (const int4*)c.hdr.p, (const float*)c.nrow.p, c.frow.p,
                          (const float*)c.props.p, c.svel.p, res, (const int*)done);
@@ -2580,8 +3027,9 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   }
   JB_CHECK(hipGetLastError());
   tEnd(c, T_SOLVE_ITER,
-       (int64_t)launchedIters * 2 *
-               (headColors - firstColor + (headColors < c.ncolors ? 1 : 0) + (blockSweeps ? 1 : 0)) +
+       (flow ? flowLaunches
+             : (int64_t)launchedIters * 2 *
+                   (headColors - firstColor + (headColors < c.ncolors ? 1 : 0) + (blockSweeps ? 1 : 0))) +
            jointLaunches);
   hipLaunchKernelGGL(kWriteback, dim3(gridFor(na)), dim3(256), 0, s, na, (const int*)nullptr, c.hdr.p, c.nrow.p, c.frow.p, man);
   hipLaunchKernelGGL(kCopyVel, dim3(gridFor(c.nb)), dim3(256), 0, s, c.nb, c.svel.p, c.vel.p, c.props.p);
@@ -2593,7 +3041,12 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   if (iters > 0)
     JB_CHECK(hipMemcpyAsync(c.solveRh.p, c.resid.p, 2 * (size_t)iters * sizeof(double), hipMemcpyDeviceToHost, s));
   JB_CHECK(hipMemcpyAsync(c.solveRows.p, c.rowCount.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+  c.flowErrHost.ensure(1);
+  c.flowErrHost.p[0] = 0;
+  if (flow)
+    JB_CHECK(hipMemcpyAsync(c.flowErrHost.p, c.flowCtl.p + kFlowCtlErr, sizeof(int), hipMemcpyDeviceToHost, s));
   c.solveStat.pending = true;
+  c.solveStat.flow = flow;
   c.solveStat.tolMode = tolMode;
   c.solveStat.blockSweeps = blockSweeps;
   c.solveStat.sampleK = sampleK;
@@ -2612,7 +3065,8 @@ void solverCollectStats(Ctx& c) {
   const unsigned long long* rowsHT = c.solveRows.p;
   c.st.rows = (int64_t)rowsHT[0];
   // rows swept per sweep by the per-colour launches (kinds 0, 1) and by the block launches (kinds 2, 3)
-  const int64_t colourRows = blockSweeps ? (int64_t)(rowsHT[0] - rowsHT[1]) : (int64_t)rowsHT[1];
+  const int64_t colourRows = blockSweeps ? (int64_t)(rowsHT[0] - rowsHT[1])
+                                         : (int64_t)rowsHT[c.solveStat.flow ? 0 : 1];
   const int64_t blockRows = blockSweeps ? (int64_t)rowsHT[1] : 0;
   if (c.solveStat.sampleK) {
     for (size_t e = 0; e < c.solveStat.kUsed; e += 2) {
@@ -2630,6 +3084,7 @@ void solverCollectStats(Ctx& c) {
   }
   c.st.residual = ro[0];
   c.st.iterations = (int64_t)ro[1];
+  if (c.solveStat.flow && c.flowErrHost.p[0]) throw std::runtime_error("a solver sweep's bounded wait gave up");
   if (c.wbLastSolve) {
     const int* wi = c.wbInfoHost.p;
     c.st.colors = wi[1];
@@ -2701,6 +3156,7 @@ void solverStatsCopy(Ctx& c) {
   c.solveStat.pending = true;
   c.solveStat.tolMode = false;
   c.solveStat.blockSweeps = false;
+  c.solveStat.flow = false;
   c.solveStat.sampleK = false;
   c.solveStat.iters = iters;
   c.solveStat.kUsed = 0;

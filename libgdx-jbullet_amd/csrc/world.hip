@@ -250,11 +250,13 @@ void bodiesToDevice(Ctx& c, const float* bodies) {
   c.bodyShapeType.resize(n);
   c.bodyStaticHost.resize(n);
   c.bodyInvMassHost.resize(n);
+  c.oddBodies = false;
   for (int i = 0; i < n; i++) {
     const float* r = bodies + (size_t)JBGPU_BODY_WORDS * i;
     c.bodyShapeType[i] = c.shapeTypeHost[ldi(r + 27)];
     c.bodyStaticHost[i] = (ldi(r + 28) & JBGPU_BODY_STATIC) != 0;
     c.bodyInvMassHost[i] = r[18];
+    if (c.bodyStaticHost[i] && r[18] != 0.0f) c.oddBodies = true;
   }
   c.wbReady = false;
   jointsChanged(c);
