@@ -179,7 +179,9 @@ struct RayTree {
   // per query
   DBuf<int> count;
   DBuf<int64_t> offset;
-  DBuf<uint64_t> keys, keysAlt;
+  DBuf<uint64_t> keys;               // candidates: query << 32 | object
+  DBuf<unsigned long long> total;    // their number, error bits
+  HBuf<unsigned long long> totalHost;
   DBuf<float> rec, io;
   DBuf<int> ioInt;
   // convex sweeps: per query the origins of from and to, then the cast shape's AABB over the sweep (12 floats),
@@ -266,7 +268,6 @@ struct Ctx {
   DBuf<unsigned long long> counter;  // misc device counters
   DBuf<int> primTmp;  // scratch of the device-wide scans, compactions and sorts (prim.hip)
   HBuf<int> primErrHost;  // the sorts' error word, read back after a step
-  DBuf<int> primWide;
   int64_t pairCap = 0;
   // pairs and manifolds (double buffered for the remap)
   int cur = 0;
@@ -541,9 +542,8 @@ void primSelectIndex(Ctx& c, const int* flag, int n, int* out, int* count);
 // out[0, m) = vals[i] for the i < n with flag[i] != 0, in index order; *count (device) = m
 template <class T>
 void primSelectValues(Ctx& c, const T* vals, const int* flag, int n, T* out, int* count);
-// out[i] = in[0] + ... + in[i - 1], i < n (the sums must fit in an int; primScanWide writes them as int64)
+// out[i] = in[0] + ... + in[i - 1], i < n (the sums must fit in an int)
 void primScan(Ctx& c, const int* in, int* out, int n);
-void primScanWide(Ctx& c, const int* in, int64_t* out, int n);
 // the same with the element count in device memory (*count, at most cap): launches shaped by cap only, as a
 // captured graph needs; the sorted data ends in k.cur / v.cur (which buffer that is depends on cap and the bits)
 void primReserve(Ctx& c, int cap);  // scratch for counts up to cap, allocated outside a capture

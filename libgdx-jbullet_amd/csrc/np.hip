@@ -1412,129 +1412,218 @@ __device__ bool rayAabb(V3 from, V3 to, V3 mn, V3 mx, float& param) {
   }
   return false;
 }
-// conservative segment-box test for tree nodes (double precision, box widened): never rejects a box that the
-// exact float test above accepts
-__device__ __forceinline__ bool segmentHitsBox(V3 F, V3 T, float4 mn, float4 mx) {
-  double t0 = 0.0, t1 = 1.0;
-  const float fo[3] = {F.x, F.y, F.z}, ft[3] = {T.x, T.y, T.z};
-  const float lo[3] = {mn.x, mn.y, mn.z}, hi[3] = {mx.x, mx.y, mx.z};
-  for (int a = 0; a < 3; a++) {
-    const double l = lo[a], h = hi[a];
-    const double eps = 1e-5 * (fabs(l) + fabs(h) + fabs((double)fo[a]) + fabs((double)ft[a])) + 1e-6;
-    const double o = fo[a], d = (double)ft[a] - (double)fo[a];
-    if (d == 0.0) {
-      if (o < l - eps || o > h + eps) return false;
-    } else {
-      double ta = (l - eps - o) / d, tb = (h + eps - o) / d;
-      if (ta > tb) {
-        const double x = ta;
-        ta = tb;
-        tb = x;
-      }
-      t0 = ta > t0 ? ta : t0;
-      t1 = tb < t1 ? tb : t1;
-      if (t0 > t1) return false;
-    }
+// conservative segment-box test for tree nodes: the box is widened by 1e-5 of the coordinates' magnitudes, two orders
+// above the rounding of this test and of the exact one, so it never rejects a box that the exact test accepts.  One
+// reciprocal per axis and query in 32 bits: the former test in 64 bits with two divisions per axis and box took most
+// of the traversal's time.
+struct Segment {
+  V3 from, inv, eps;
+  bool flat[3];  // no motion along the axis
+};
+__device__ __forceinline__ Segment makeSegment(V3 F, V3 T) {
+  Segment s;
+  const V3 d = sub(T, F);
+  s.from = F;
+  s.flat[0] = fabsf(d.x) < 1e-30f;
+  s.flat[1] = fabsf(d.y) < 1e-30f;
+  s.flat[2] = fabsf(d.z) < 1e-30f;
+  s.inv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+  s.eps = v3(1e-5f * (fabsf(F.x) + fabsf(T.x)) + 1e-6f, 1e-5f * (fabsf(F.y) + fabsf(T.y)) + 1e-6f,
+             1e-5f * (fabsf(F.z) + fabsf(T.z)) + 1e-6f);
+  return s;
+}
+__device__ __forceinline__ void segmentAxis(float lo, float hi, float from, float inv, float eps, bool flat, float& t0,
+                                            float& t1) {
+  const float e = 1e-5f * (fabsf(lo) + fabsf(hi)) + eps;
+  const float a = (lo - e) - from, b = (hi + e) - from;
+  if (flat) {
+    if (a > 0.0f || b < 0.0f) t1 = -1.0f;
+    return;
   }
-  return true;
+  const float ta = a * inv, tb = b * inv;
+  t0 = fmaxf(t0, fminf(ta, tb));
+  t1 = fminf(t1, fmaxf(ta, tb));
+}
+__device__ __forceinline__ bool segmentHitsBox(const Segment& s, float4 mn, float4 mx) {
+  float t0 = 0.0f, t1 = 1.0f;
+  segmentAxis(mn.x, mx.x, s.from.x, s.inv.x, s.eps.x, s.flat[0], t0, t1);
+  segmentAxis(mn.y, mx.y, s.from.y, s.inv.y, s.eps.y, s.flat[1], t0, t1);
+  segmentAxis(mn.z, mx.z, s.from.z, s.inv.z, s.eps.z, s.flat[2], t0, t1);
+  return !(t0 > t1);
 }
 __device__ __forceinline__ bool rayNeeds(int filt, int group, int mask) {  // RayResultCallback.needsCollision
   const int pg = (int)(short)(filt & 0xffff), pm = (int)(short)(filt >> 16);
   return ((pg & mask) & 0xFFFF) != 0 && ((group & pm) & 0xFFFF) != 0;
 }
 
-// candidate objects of every ray: filter and rayAabb with the callback's initial fraction (1); the count pass
-// stores the number per ray, the emit pass writes (ray << 32 | object) at the ray's offset.  With `expand`
-// (min xyz, max xyz: a convex sweep's cast-shape AABB) every object box is widened by it first, as
-// AabbUtil2.aabbExpand does (node boxes alike: float addition keeps them around their leaves).  A query's
-// from, to and expand values start at stride * query.
-constexpr int kRayStack = 64;
-template <bool Emit>
-__global__ void kRayCandidates(int nr, const float* __restrict__ from, const float* __restrict__ to,
-                               const float* __restrict__ expand, int stride,
-                               const int* __restrict__ rworld, int group, int mask, int nn,
-                               const float4* __restrict__ rec, const int4* __restrict__ leafExact,
-                               const int* __restrict__ hugeRange, const int* __restrict__ hugeList,
-                               const float* __restrict__ aabb, const int* __restrict__ filt,
-                               const int* __restrict__ wid, int maxWorld, int* count,
-                               const int64_t* __restrict__ offset, uint64_t* keys, int* err) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nr) return;
-  const float* fp = from + (size_t)stride * r;
-  const float* tp = to + (size_t)stride * r;
-  const V3 F = v3(fp[0], fp[1], fp[2]), T = v3(tp[0], tp[1], tp[2]);
-  V3 emn = v3(0, 0, 0), emx = v3(0, 0, 0);
-  if (expand) {
-    const float* ep = expand + (size_t)stride * r;
-    emn = v3(ep[0], ep[1], ep[2]);
-    emx = v3(ep[3], ep[4], ep[5]);
-  }
-  const int w = rworld ? rworld[r] : 0;
-  if (w < 0 || w > maxWorld) {  // a world id the proxies never had: no candidates, and the call reports it
-    if (!Emit) {
-      count[r] = 0;
-      atomicOr(err, 2);
+// Candidate objects of every query (ray or convex sweep): filter and rayAabb with the callback's initial fraction (1).
+// G lanes share a query: they pop up to G nodes off the query's stack in LDS, each tests its node's two children and
+// pushes the inner ones that the segment meets; leaves are tested exactly and collected in LDS.  The block then takes
+// one contiguous range of the candidate array for all its queries (one atomic per block) and writes (query << 32 |
+// object); a query with more than its LDS share walks its tree again and writes directly.  One traversal where a
+// counting pass, a scan and an emitting pass with one lane per query took two, and a wave's worth of lanes where few
+// queries would leave the chip idle: 4099 sweeps over 5005 bodies 11.0 -> 0.19 ms, 262,144 rays over 20,005 bodies
+// 5.4 (with the sort by object that the fold no longer needs) -> 0.9 ms.  With `expand` (min xyz, max xyz: a sweep's
+// cast-shape AABB) every object box is widened by it first, as AabbUtil2.aabbExpand does (node boxes alike: float
+// addition keeps them around their leaves).  A query's from, to and expand values start at stride * query.  total:
+// entries asked for so far; nothing is written past cap.
+constexpr int kQueryBlock = 256;
+constexpr int kQueryWide = 1 << 14;  // from this many queries on, half a wave each
+constexpr int kQueryReserve = 128;  // stack entries kept for a plain descent: more than the deepest tree
+template <int G, int Stack, int Share>
+__global__ __launch_bounds__(kQueryBlock) void kQueryCandidates(
+    int nr, const float* __restrict__ from, const float* __restrict__ to, const float* __restrict__ expand, int stride,
+    const int* __restrict__ rworld, int group, int mask, int nn, const float4* __restrict__ rec,
+    const int4* __restrict__ leafExact, const int* __restrict__ hugeRange, const int* __restrict__ hugeList,
+    const float* __restrict__ aabb, const int* __restrict__ filt, const int* __restrict__ wid, int maxWorld, int* count,
+    int64_t* offset, uint64_t* keys, int64_t cap, unsigned long long* total, int* err) {
+  constexpr int Q = kQueryBlock / G;  // queries per block
+  static_assert(Stack >= kQueryReserve + 2 * G, "room for one wide step above the reserve");
+  __shared__ int stackLds[Q][Stack];
+  __shared__ int candLds[Q][Share];
+  __shared__ int countLds[Q];
+  __shared__ unsigned long long baseLds;
+  const int qi = threadIdx.x / G, gl = threadIdx.x % G;
+  const int lane = threadIdx.x & 63;
+  const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << (G & 63)) - 1)) << (lane - gl);
+  const unsigned long long below = gmask & ((1ull << lane) - 1);
+  const int r = blockIdx.x * Q + qi;
+  int* const stack = stackLds[qi];
+  int* const mine = candLds[qi];
+  int w = 0;
+  bool active = r < nr;
+  V3 F = v3(0, 0, 0), T = v3(0, 0, 0), emn = v3(0, 0, 0), emx = v3(0, 0, 0);
+  if (active) {
+    const float* fp = from + (size_t)stride * r;
+    const float* tp = to + (size_t)stride * r;
+    F = v3(fp[0], fp[1], fp[2]);
+    T = v3(tp[0], tp[1], tp[2]);
+    if (expand) {
+      const float* ep = expand + (size_t)stride * r;
+      emn = v3(ep[0], ep[1], ep[2]);
+      emx = v3(ep[3], ep[4], ep[5]);
     }
-    return;
+    w = rworld ? rworld[r] : 0;
+    if (w < 0 || w > maxWorld) {  // a world id the proxies never had: no candidates, and the call reports it
+      atomicOr(err, 2);
+      active = false;
+    }
   }
-  int cnt = 0;
-  const int64_t base = Emit ? offset[r] : 0;
-  const int room = Emit ? count[r] : 0;  // the emit pass writes no more than the count pass found
-  auto consider = [&](int o, V3 mn, V3 mx, int f) {
-    if (wid[o] != w || !rayNeeds(f, group, mask)) return;  // other worlds are other collision-object lists
+  const Segment seg = makeSegment(F, T);
+  auto hits = [&](int o, V3 mn, V3 mx, int f) {
+    if (wid[o] != w || !rayNeeds(f, group, mask)) return false;  // other worlds are other collision-object lists
     if (expand) {
       mn = add(mn, emn);
       mx = add(mx, emx);
     }
     float param = 1.0f;
-    if (!rayAabb(F, T, mn, mx, param)) return;
-    if (Emit && cnt < room) keys[base + cnt] = ((uint64_t)(uint32_t)r << 32) | (uint32_t)o;
-    cnt++;
+    return rayAabb(F, T, mn, mx, param);
   };
-  for (int k = hugeRange[2 * w]; k < hugeRange[2 * w + 1]; k++) {
-    const int o = hugeList[k];
-    const float* A = aabb + 6 * o;
-    consider(o, v3(A[0], A[1], A[2]), v3(A[3], A[4], A[5]), filt[o]);
-  }
-  auto leaf = [&](int t) {
+  auto leafHits = [&](int t, int& o) {
     const int4 e0 = leafExact[2 * t], e1 = leafExact[2 * t + 1];
-    consider(e1.w, v3(__int_as_float(e0.x), __int_as_float(e0.y), __int_as_float(e0.z)),
-             v3(__int_as_float(e0.w), __int_as_float(e1.x), __int_as_float(e1.y)), e1.z);
+    o = e1.w;
+    return hits(o, v3(__int_as_float(e0.x), __int_as_float(e0.y), __int_as_float(e0.z)),
+                v3(__int_as_float(e0.w), __int_as_float(e1.x), __int_as_float(e1.y)), e1.z);
   };
-  if (nn == 1) {
-    leaf(0);
-  } else if (nn >= 2) {
-    int stack[kRayStack];
-    int sp = 0, node = 0;
-    while (true) {
-      const float4* R = rec + kRecF4 * node;
-      const float4 m = R[4];
-      int next = -1;
-      for (int c = 0; c < 2; c++) {
-        const int ch = __float_as_int(c == 0 ? m.x : m.y);
-        float4 bmn = R[2 * c], bmx = R[2 * c + 1];
-        if (w < __float_as_int(bmn.w) || w > __float_as_int(bmx.w)) continue;
-        if (expand) {
-          bmn.x += emn.x; bmn.y += emn.y; bmn.z += emn.z;
-          bmx.x += emx.x; bmx.y += emx.y; bmx.z += emx.z;
-        }
-        if (!segmentHitsBox(F, T, bmn, bmx)) continue;
-        if (ch < 0) {
-          leaf(-ch - 1);
-        } else if (next < 0) {
-          next = ch;
-        } else if (sp < kRayStack) {
-          stack[sp++] = ch;
-        } else {
-          atomicOr(err, 1);
-        }
+  // the query's candidates, handed to put(index, object) in any order; returns their number (group-uniform)
+  auto walk = [&](auto put) {
+    int n = 0;
+    auto collect = [&](bool hit, int o) {
+      const unsigned long long m = __ballot(hit) & gmask;
+      if (hit) put(n + __popcll(m & below), o);
+      n += __popcll(m);
+    };
+    const int h1 = hugeRange[2 * w + 1];
+    for (int k0 = hugeRange[2 * w]; k0 < h1; k0 += G) {
+      const int k = k0 + gl;
+      bool hit = false;
+      int o = 0;
+      if (k < h1) {
+        o = hugeList[k];
+        const float* A = aabb + 6 * o;
+        hit = hits(o, v3(A[0], A[1], A[2]), v3(A[3], A[4], A[5]), filt[o]);
       }
-      if (next >= 0) node = next;
-      else if (sp > 0) node = stack[--sp];
-      else break;
+      collect(hit, o);
     }
+    if (nn == 1) {
+      int o = 0;
+      const bool hit = gl == 0 && leafHits(0, o);
+      collect(hit, o);
+    }
+    int size = 0;
+    if (nn >= 2) {
+      if (gl == 0) stack[0] = 0;
+      size = 1;
+    }
+    while (size > 0) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the last step's pushes
+      // wide steps while the stack holds them above the reserve, else one node at a time (a plain descent)
+      const int wide = min(min(size, G), Stack - kQueryReserve - size);
+      const int pop = max(wide, 1);
+      const bool on = gl < pop;
+      const int node = on ? stack[size - 1 - gl] : 0;
+      size -= pop;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read before this step's pushes
+      float4 b0 = make_float4(0, 0, 0, 0), b1 = b0, b2 = b0, b3 = b0, m = b0;
+      if (on) {
+        const float4* R = rec + kRecF4 * (size_t)node;
+        b0 = R[0]; b1 = R[1]; b2 = R[2]; b3 = R[3]; m = R[4];
+      }
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        float4 bmn = c == 0 ? b0 : b2, bmx = c == 0 ? b1 : b3;
+        const int ch = __float_as_int(c == 0 ? m.x : m.y);
+        bool meets = on && w >= __float_as_int(bmn.w) && w <= __float_as_int(bmx.w);
+        if (meets) {
+          if (expand) {
+            bmn.x += emn.x; bmn.y += emn.y; bmn.z += emn.z;
+            bmx.x += emx.x; bmx.y += emx.y; bmx.z += emx.z;
+          }
+          meets = segmentHitsBox(seg, bmn, bmx);
+        }
+        const unsigned long long inner = __ballot(meets && ch >= 0) & gmask;
+        if (meets && ch >= 0) {
+          const int at = size + __popcll(inner & below);
+          if (at < Stack) stack[at] = ch;
+          else atomicOr(err, 1);
+        }
+        size = min(size + __popcll(inner), Stack);
+        int o = 0;
+        const bool hit = meets && ch < 0 && leafHits(-ch - 1, o);
+        collect(hit, o);
+      }
+    }
+    return n;
+  };
+  int n = 0;
+  if (active)
+    n = walk([&](int at, int o) {
+      if (at < Share) mine[at] = o;
+    });
+  if (gl == 0) countLds[qi] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long sum = 0;
+    for (int k = 0; k < Q; k++) sum += (unsigned long long)countLds[k];
+    baseLds = sum ? atomicAdd(total, sum) : 0ull;
   }
-  if (!Emit) count[r] = cnt;
+  __syncthreads();
+  if (r >= nr) return;
+  int64_t base = (int64_t)baseLds;
+  for (int k = 0; k < qi; k++) base += countLds[k];
+  if (gl == 0) {
+    count[r] = n;
+    offset[r] = base;
+  }
+  if (n == 0 || base + n > cap) return;
+  const uint64_t hi = (uint64_t)(uint32_t)r << 32;
+  if (n <= Share) {
+    for (int k = gl; k < n; k += G) keys[base + k] = hi | (uint32_t)mine[k];
+  } else {
+    walk([&](int at, int o) {
+      if (at < n) keys[base + at] = hi | (uint32_t)o;
+    });
+  }
 }
 
 // planeSpace1 (TransformUtil.java:45-61)
@@ -1625,14 +1714,15 @@ __device__ bool subsimplexRayCast(Simplex& ss, const Shape& sb, const float* ver
   return true;
 }
 
-// per candidate (sorted by ray, then object): the object's hit, independent of the ray's running fraction.
-// record: [flags (bit0 hit / first triangle, bit1 second triangle, bit2 plane), f0, n0 xyz, f1, n1 xyz, -]
-constexpr int kRayRec = 10;
+// per candidate: the object's hit, independent of the ray's running fraction.
+// record: [flags (bit0 hit / first triangle, bit1 second triangle, bit2 plane), f0, f1, entry, n0 xyz, -, n1 xyz, -]
+constexpr int kRayRec = 12;
 __global__ __launch_bounds__(kGjkBlock) void kRayCast(int64_t n, const uint64_t* __restrict__ keys,
                                                       const float* __restrict__ from, const float* __restrict__ to,
                                                       const float* __restrict__ shapes,
                                                       const float* __restrict__ props, const float* __restrict__ tr,
-                                                      const float* __restrict__ verts, float* out) {
+                                                      const float* __restrict__ verts,
+                                                      const float* __restrict__ aabb, float* out) {
   __shared__ float simplexLds[kSimplexRows * kGjkBlock];
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -1676,48 +1766,82 @@ __global__ __launch_bounds__(kGjkBlock) void kRayCast(int64_t n, const uint64_t*
       n1 = mulMV(tb.b, nl);
     }
   }
-  R[0] = __int_as_float(flags);
-  R[1] = f0;
-  R[2] = n0.x; R[3] = n0.y; R[4] = n0.z;
-  R[5] = f1;
-  R[6] = n1.x; R[7] = n1.y; R[8] = n1.z;
-  R[9] = 0.0f;
+  float entry = 1.0f;  // where the ray enters the object's AABB
+  if (flags & 3) {
+    const float* A = aabb + 6 * o;
+    rayAabb(F, T, v3(A[0], A[1], A[2]), v3(A[3], A[4], A[5]), entry);
+  }
+  ((float4*)R)[0] = make_float4(__int_as_float(flags), f0, f1, entry);
+  if (flags & 3) {
+    ((float4*)R)[1] = make_float4(n0.x, n0.y, n0.z, 0.0f);
+    ((float4*)R)[2] = make_float4(n1.x, n1.y, n1.z, 0.0f);
+  }
 }
 
 // ClosestRayResultCallback over a ray's candidates in world order: rayAabb with the running fraction, then
-// the object's hit if its fraction is below it (CollisionWorld.java:566-589, :282-298, :710-727)
+// the object's hit if its fraction is below it (CollisionWorld.java:566-589, :282-298, :710-727).  A candidate's AABB
+// meets the ray, so with the running fraction it still does unless it is entered past that.  kFoldLanes lanes
+// share a ray; its candidates lie in any order, and an object that changes nothing can be passed over: each round the
+// lanes find the lowest object after the last that would change the running fraction, and apply it.
+constexpr int kFoldLanes = 8;
+__device__ __forceinline__ int foldMin(int x) {  // over a query's lanes
+  for (int off = 1; off < kFoldLanes; off <<= 1) x = min(x, __shfl_xor(x, off));
+  return x;
+}
 __global__ void kRayFold(int nr, const int* __restrict__ count, const int64_t* __restrict__ offset,
                          const uint64_t* __restrict__ keys, const float* __restrict__ recs,
-                         const float* __restrict__ from, const float* __restrict__ to,
-                         const float* __restrict__ aabb, int* obj, float* frac, float* normal, float* point) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+                         const float* __restrict__ from, const float* __restrict__ to, int* obj, float* frac,
+                         float* normal, float* point) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int r = t / kFoldLanes, gl = t % kFoldLanes;
   if (r >= nr) return;
   const V3 F = v3(from[3 * r], from[3 * r + 1], from[3 * r + 2]), T = v3(to[3 * r], to[3 * r + 1], to[3 * r + 2]);
   float best = 1.0f;
-  int hit = -1;
+  int hit = -1, last = -1;
   V3 hn = v3(0, 0, 0), hp = v3(0, 0, 0);
   const int64_t b = offset[r], e = b + count[r];
-  for (int64_t k = b; k < e; k++) {
-    if (best == 0.0f) break;
-    const int o = (int)(keys[k] & 0xffffffffu);
-    const float* A = aabb + 6 * o;
-    float param = best;
-    if (!rayAabb(F, T, v3(A[0], A[1], A[2]), v3(A[3], A[4], A[5]), param)) continue;
+  // each lane keeps its first candidate (most rays have no more than kFoldLanes)
+  uint64_t key0 = 0;
+  float4 rec0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (b + gl < e) {
+    key0 = keys[b + gl];
+    rec0 = *(const float4*)(recs + kRayRec * (b + gl));
+  }
+  while (best != 0.0f) {
+    int next = 0x7fffffff;
+    int64_t at = b;
+    for (int64_t k = b + gl; k < e; k += kFoldLanes) {
+      const int o = (int)((k == b + gl ? key0 : keys[k]) & 0xffffffffu);
+      if (o <= last || o >= next) continue;
+      const float4 R = k == b + gl ? rec0 : *(const float4*)(recs + kRayRec * k);
+      const int flags = __float_as_int(R.x);
+      if (!((flags & 1) && R.y < best) && !((flags & 2) && R.z < best)) continue;
+      if (!(R.w <= best)) continue;  // rayAabb with the running fraction
+      next = o;
+      at = k;
+    }
+    const int first = foldMin(next);
+    if (first == 0x7fffffff) break;
+    // the lane that holds it hands its record's place to the others
+    const int owner = foldMin(next == first ? gl : kFoldLanes);
+    const int64_t k = b + __shfl((int)(at - b), owner, kFoldLanes);
     const float* R = recs + kRayRec * k;
     const int flags = __float_as_int(R[0]);
+    last = first;
     if ((flags & 1) && R[1] < best) {
       best = R[1];
-      hit = o;
-      hn = v3(R[2], R[3], R[4]);
+      hit = first;
+      hn = v3(R[4], R[5], R[6]);
       hp = interp3(F, T, best);
     }
-    if ((flags & 2) && R[5] < best) {  // the plane's second triangle, against the updated fraction
-      best = R[5];
-      hit = o;
-      hn = v3(R[6], R[7], R[8]);
+    if ((flags & 2) && R[2] < best) {  // the plane's second triangle, against the updated fraction
+      best = R[2];
+      hit = first;
+      hn = v3(R[8], R[9], R[10]);
       hp = interp3(F, T, best);
     }
   }
+  if (gl) return;
   obj[r] = hit;
   frac[r] = best;
   normal[3 * r] = hn.x; normal[3 * r + 1] = hn.y; normal[3 * r + 2] = hn.z;
@@ -1875,7 +1999,7 @@ __global__ void kSweepPrep(int nq, const float* __restrict__ castRec, const floa
   st3(o + 9, mx);
 }
 
-// per candidate (sorted by query, then object): objectQuerySingle's convex branch (CollisionWorld.java:392-424)
+// per candidate: objectQuerySingle's convex branch (CollisionWorld.java:392-424)
 // up to the fraction test: the cast with allowedCcdPenetration 0.04 and a normal longer than 0.01, normalised.
 // Planes are not convex and have no caster there: never a hit.  record: [hit, fraction, normal xyz, point xyz]
 constexpr int kSweepRec = 8;
@@ -1910,25 +2034,43 @@ __global__ __launch_bounds__(kGjkBlock) void kSweepCast(int64_t n, const uint64_
   st3(R + 5, pt);
 }
 
-// ClosestConvexResultCallback over a query's candidates in world order: a hit below the running fraction
-// replaces it (CollisionWorld.java:766-810)
+// ClosestConvexResultCallback over a query's candidates: in world order a hit below the running fraction replaces it
+// (CollisionWorld.java:766-810), so the smallest fraction below 1 stays, at its lowest object
 __global__ void kSweepFold(int nq, const int* __restrict__ count, const int64_t* __restrict__ offset,
                            const uint64_t* __restrict__ keys, const float* __restrict__ recs, int* obj, float* frac,
                            float* normal, float* point) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int q = t / kFoldLanes, gl = t % kFoldLanes;
   if (q >= nq) return;
   float best = 1.0f;
   int hit = -1;
-  V3 hn = v3(0, 0, 0), hp = v3(0, 0, 0);
   const int64_t b = offset[q], e = b + count[q];
-  for (int64_t k = b; k < e; k++) {
+  int64_t at = b;
+  for (int64_t k = b + gl; k < e; k += kFoldLanes) {
     const float* R = recs + kSweepRec * k;
-    if (R[0] != 0.0f && R[1] < best) {
+    const int o = (int)(keys[k] & 0xffffffffu);
+    if (R[0] != 0.0f && (R[1] < best || (R[1] == best && hit >= 0 && o < hit))) {
       best = R[1];
-      hit = (int)(keys[k] & 0xffffffffu);
-      hn = v3(R[2], R[3], R[4]);
-      hp = v3(R[5], R[6], R[7]);
+      hit = o;
+      at = k;
     }
+  }
+  int64_t place = at - b;
+  for (int off = 1; off < kFoldLanes; off <<= 1) {
+    const float f = __shfl_xor(best, off);
+    const int h = __shfl_xor(hit, off), p = __shfl_xor((int)place, off);
+    if (h >= 0 && (hit < 0 || f < best || (f == best && h < hit))) {
+      best = f;
+      hit = h;
+      place = p;
+    }
+  }
+  if (gl) return;
+  V3 hn = v3(0, 0, 0), hp = v3(0, 0, 0);
+  if (hit >= 0) {
+    const float* R = recs + kSweepRec * (b + place);
+    hn = v3(R[2], R[3], R[4]);
+    hp = v3(R[5], R[6], R[7]);
   }
   obj[q] = hit;
   frac[q] = best;
@@ -2178,57 +2320,60 @@ void npCollectStats(Ctx& c) {  // after the step's final synchronisation
 }
 
 
+// the candidates of n queries into t.keys (contiguous per query: t.offset, t.count); returns their number.  The array
+// keeps its size from call to call; a call that needs more has counted them and walks again with enough.
+static int64_t queryCandidates(Ctx& c, int n, const float* from, const float* to, const float* expand, int stride,
+                               const int* dWorld, int16_t group, int16_t mask, const char* what) {
+  RayTree& t = c.rt;
+  hipStream_t s = c.stream;
+  t.count.ensure(n);
+  t.offset.ensure(n);
+  t.keys.ensure(8 * (size_t)n);
+  // [0] candidates, [1] error bits
+  t.total.ensure(2);
+  t.totalHost.ensure(2);
+  for (;;) {
+    const int64_t cap = (int64_t)t.keys.n;
+    JB_CHECK(hipMemsetAsync(t.total.p, 0, 2 * sizeof(unsigned long long), s));
+    auto launch = [&](auto kernel, int lanes) {
+      hipLaunchKernelGGL(kernel, dim3(gridFor((int64_t)n * lanes, kQueryBlock)), dim3(kQueryBlock), 0, s, n, from, to,
+                         expand, stride, dWorld, (int)group, (int)mask, t.nn, (const float4*)t.nodeRec.p,
+                         (const int4*)t.leafExact.p, (const int*)t.hugeRange.p, (const int*)t.hugeList.p,
+                         (const float*)t.aabb.p, (const int*)c.filt.p, (const int*)c.world.p, c.maxWorld, t.count.p,
+                         t.offset.p, t.keys.p, cap, t.total.p, (int*)(t.total.p + 1));
+    };
+    // A wave per query until the queries alone fill the chip, then half a wave.  Whole calls over a 20,005-body pile,
+    // 16 / 32 / 64 lanes a query: 1000 rays 661 / 486 / 465 us, 16,000 689 / 559 / 562 us, 60,000 1002 / 913 / - us,
+    // 262,144 2543 / 2588 / - us (8 lanes 3063, 4 lanes 4997); 4099 sweeps over 5005 bodies 2844 / 2588 / 2427 us.
+    if (n < kQueryWide) launch(kQueryCandidates<64, 768, 512>, 64);
+    else launch(kQueryCandidates<32, 384, 128>, 32);
+    JB_CHECK(hipMemcpyAsync(t.totalHost.p, t.total.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    JB_CHECK(hipStreamSynchronize(s));
+    const int err = (int)t.totalHost.p[1];
+    if (err & 2) throw std::invalid_argument(std::string(what) + " world id out of range (no such world among the proxies)");
+    if (err & 1) throw std::runtime_error(std::string(what) + " traversal stack overflow");
+    const int64_t total = (int64_t)t.totalHost.p[0];
+    if (total >= (int64_t)1 << 31) throw std::length_error(std::string("too many ") + what + " candidates in one call");
+    if (total <= cap) return total;
+    t.keys.ensure((size_t)total);
+  }
+}
+
 void rayTest(Ctx& c, int n, const float* dFrom, const float* dTo, int16_t group, int16_t mask, const int* dWorld,
              int* dObj, float* dFrac, float* dNormal, float* dPoint) {
   if (n <= 0) return;
   rayBuildTree(c);
   RayTree& t = c.rt;
   hipStream_t s = c.stream;
-  t.count.ensure((size_t)n + 1);  // count[n] = 0 closes the scan: offset[n] is the total
-  t.offset.ensure((size_t)n + 1);
-  int* err = (int*)(c.counter.p + 6);
-  JB_CHECK(hipMemsetAsync(err, 0, sizeof(int), s));
-  hipLaunchKernelGGL(kRayCandidates<false>, dim3(gridFor(n)), dim3(256), 0, s, n, dFrom, dTo, (const float*)nullptr, 3,
-                     dWorld, (int)group,
-                     (int)mask, t.nn, (const float4*)t.nodeRec.p, (const int4*)t.leafExact.p, (const int*)t.hugeRange.p,
-                     (const int*)t.hugeList.p, (const float*)t.aabb.p, (const int*)c.filt.p,
-                     (const int*)c.world.p, c.maxWorld, t.count.p, (const int64_t*)nullptr, (uint64_t*)nullptr, err);
-  JB_CHECK(hipMemsetAsync(t.count.p + n, 0, sizeof(int), s));
-  primScanWide(c, t.count.p, t.offset.p, n + 1);
-  int64_t total = 0;
-  int errh = 0;
-  JB_CHECK(hipMemcpyAsync(&total, t.offset.p + n, sizeof(total), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(&errh, err, sizeof(int), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipStreamSynchronize(s));
-  if (errh & 2) throw std::invalid_argument("ray world id out of range (no such world among the proxies)");
-  if (errh & 1) throw std::runtime_error("ray traversal stack overflow");
-  if (total > 0) {
-    t.keys.ensure(total);
-    t.keysAlt.ensure(total);
-    t.rec.ensure((size_t)kRayRec * total);
-    hipLaunchKernelGGL(kRayCandidates<true>, dim3(gridFor(n)), dim3(256), 0, s, n, dFrom, dTo, (const float*)nullptr, 3,
-                       dWorld, (int)group,
-                       (int)mask, t.nn, (const float4*)t.nodeRec.p, (const int4*)t.leafExact.p,
-                       (const int*)t.hugeRange.p, (const int*)t.hugeList.p, (const float*)t.aabb.p,
-                       (const int*)c.filt.p, (const int*)c.world.p, c.maxWorld, t.count.p, (const int64_t*)t.offset.p,
-                       t.keys.p, err);
-    // world order inside every ray's segment: sort by (ray, object)
-    int bits = 32;
-    while (bits < 64 && (1ll << (bits - 32)) < (int64_t)n) bits++;
-    if (total >= (int64_t)1 << 31) throw std::length_error("too many ray candidates in one call");
-    Db<uint64_t> kk(t.keys.p, t.keysAlt.p);
-    primSortKeys(c, kk, (int)total, 0, bits);
+  const int64_t total = queryCandidates(c, n, dFrom, dTo, nullptr, 3, dWorld, group, mask, "ray");
+  t.rec.ensure((size_t)kRayRec * std::max<int64_t>(total, 1));
+  if (total > 0)
     hipLaunchKernelGGL(kRayCast, dim3(gridFor(total, kGjkBlock)), dim3(kGjkBlock), 0, s, total,
-                       (const uint64_t*)kk.Current(), dFrom, dTo, (const float*)c.shapes.p, (const float*)c.props.p,
-                       (const float*)c.tr.p, (const float*)c.verts.p, t.rec.p);
-    hipLaunchKernelGGL(kRayFold, dim3(gridFor(n)), dim3(256), 0, s, n, (const int*)t.count.p,
-                       (const int64_t*)t.offset.p, (const uint64_t*)kk.Current(), (const float*)t.rec.p, dFrom, dTo,
-                       (const float*)t.aabb.p, dObj, dFrac, dNormal, dPoint);
-  } else {
-    hipLaunchKernelGGL(kRayFold, dim3(gridFor(n)), dim3(256), 0, s, n, (const int*)t.count.p,
-                       (const int64_t*)t.offset.p, (const uint64_t*)nullptr, (const float*)nullptr, dFrom, dTo,
-                       (const float*)t.aabb.p, dObj, dFrac, dNormal, dPoint);
-  }
+                       (const uint64_t*)t.keys.p, dFrom, dTo, (const float*)c.shapes.p, (const float*)c.props.p,
+                       (const float*)c.tr.p, (const float*)c.verts.p, (const float*)t.aabb.p, t.rec.p);
+  hipLaunchKernelGGL(kRayFold, dim3(gridFor((int64_t)n * kFoldLanes)), dim3(256), 0, s, n, (const int*)t.count.p,
+                     (const int64_t*)t.offset.p, (const uint64_t*)t.keys.p, (const float*)t.rec.p, dFrom, dTo, dObj,
+                     dFrac, dNormal, dPoint);
 }
 
 void sweepTest(Ctx& c, int n, const float* castShape, const float* dFrom, const float* dTo, int16_t group,
@@ -2244,46 +2389,15 @@ void sweepTest(Ctx& c, int n, const float* castShape, const float* dFrom, const 
   hipLaunchKernelGGL(kSweepPrep, dim3(gridFor(n)), dim3(256), 0, s, n, (const float*)t.sweepShape.p, dFrom, dTo,
                      t.sweep.p);
   const float* F = t.sweep.p;
-  t.count.ensure((size_t)n + 1);
-  t.offset.ensure((size_t)n + 1);
-  int* err = (int*)(c.counter.p + 6);
-  JB_CHECK(hipMemsetAsync(err, 0, sizeof(int), s));
-  hipLaunchKernelGGL(kRayCandidates<false>, dim3(gridFor(n)), dim3(256), 0, s, n, F, F + 3, F + 6, 12, dWorld,
-                     (int)group, (int)mask, t.nn, (const float4*)t.nodeRec.p, (const int4*)t.leafExact.p,
-                     (const int*)t.hugeRange.p, (const int*)t.hugeList.p, (const float*)t.aabb.p,
-                     (const int*)c.filt.p, (const int*)c.world.p, c.maxWorld, t.count.p, (const int64_t*)nullptr,
-                     (uint64_t*)nullptr, err);
-  JB_CHECK(hipMemsetAsync(t.count.p + n, 0, sizeof(int), s));
-  primScanWide(c, t.count.p, t.offset.p, n + 1);
-  int64_t total = 0;
-  int errh = 0;
-  JB_CHECK(hipMemcpyAsync(&total, t.offset.p + n, sizeof(total), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(&errh, err, sizeof(int), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipStreamSynchronize(s));
-  if (errh & 2) throw std::invalid_argument("sweep world id out of range (no such world among the proxies)");
-  if (errh & 1) throw std::runtime_error("sweep traversal stack overflow");
-  if (total >= (int64_t)1 << 31) throw std::length_error("too many sweep candidates in one call");
-  const uint64_t* keys = nullptr;
-  if (total > 0) {
-    t.keys.ensure(total);
-    t.keysAlt.ensure(total);
-    t.rec.ensure((size_t)kSweepRec * total);
-    hipLaunchKernelGGL(kRayCandidates<true>, dim3(gridFor(n)), dim3(256), 0, s, n, F, F + 3, F + 6, 12, dWorld,
-                       (int)group, (int)mask, t.nn, (const float4*)t.nodeRec.p, (const int4*)t.leafExact.p,
-                       (const int*)t.hugeRange.p, (const int*)t.hugeList.p, (const float*)t.aabb.p,
-                       (const int*)c.filt.p, (const int*)c.world.p, c.maxWorld, t.count.p,
-                       (const int64_t*)t.offset.p, t.keys.p, err);
-    int bits = 32;
-    while (bits < 64 && (1ll << (bits - 32)) < (int64_t)n) bits++;
-    Db<uint64_t> kk(t.keys.p, t.keysAlt.p);
-    primSortKeys(c, kk, (int)total, 0, bits);
-    keys = kk.Current();
-    hipLaunchKernelGGL(kSweepCast, dim3(gridFor(total, kGjkBlock)), dim3(kGjkBlock), 0, s, total, keys,
-                       (const float*)t.sweepShape.p, dFrom, dTo, (const float*)c.shapes.p, (const float*)c.props.p,
-                       (const float*)c.tr.p, (const float*)c.verts.p, t.rec.p);
-  }
-  hipLaunchKernelGGL(kSweepFold, dim3(gridFor(n)), dim3(256), 0, s, n, (const int*)t.count.p,
-                     (const int64_t*)t.offset.p, keys, (const float*)t.rec.p, dObj, dFrac, dNormal, dPoint);
+  const int64_t total = queryCandidates(c, n, F, F + 3, F + 6, 12, dWorld, group, mask, "sweep");
+  t.rec.ensure((size_t)kSweepRec * std::max<int64_t>(total, 1));
+  if (total > 0)
+    hipLaunchKernelGGL(kSweepCast, dim3(gridFor(total, kGjkBlock)), dim3(kGjkBlock), 0, s, total,
+                       (const uint64_t*)t.keys.p, (const float*)t.sweepShape.p, dFrom, dTo, (const float*)c.shapes.p,
+                       (const float*)c.props.p, (const float*)c.tr.p, (const float*)c.verts.p, t.rec.p);
+  hipLaunchKernelGGL(kSweepFold, dim3(gridFor((int64_t)n * kFoldLanes)), dim3(256), 0, s, n, (const int*)t.count.p,
+                     (const int64_t*)t.offset.p, (const uint64_t*)t.keys.p, (const float*)t.rec.p, dObj, dFrac, dNormal,
+                     dPoint);
 }
 
 void ccdClamp(Ctx& c, float dt, const int* abortFlag, const int* dnp) {

@@ -552,15 +552,4 @@ void graphFill(hipStream_t s, void* p, size_t words, uint32_t v) {
   hipLaunchKernelGGL(kFill32, dim3(grid), dim3(256), 0, s, words, (uint32_t*)p, v);
 }
 
-__global__ void kWiden(int n, const int* __restrict__ in, int64_t* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = in[i];
-}
-void primScanWide(Ctx& c, const int* in, int64_t* out, int n) {
-  if (n <= 0) return;
-  c.primWide.ensure(n);
-  primExclusiveScan(c.stream, in, c.primWide.p, nullptr, n, n, primScanScratch(c, n), nullptr);
-  hipLaunchKernelGGL(kWiden, dim3(gridFor(n)), dim3(256), 0, c.stream, n, (const int*)c.primWide.p, out);
-}
-
 }  // namespace jbg

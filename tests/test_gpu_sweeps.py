@@ -120,3 +120,31 @@ def test_island_list_with_a_static_pair():
         ctx.close()
     assert np.array_equal(got[0][0].view(np.uint32), got[1][0].view(np.uint32))
     assert np.array_equal(got[0][1].view(np.uint32), got[1][1].view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 3, 64, 65, 16383, 16384, 16385])
+def test_ray_counts_around_the_lane_split(n):
+    """A ray's result does not depend on how many rays are asked for: a wave per ray below 16,384 rays, half a wave
+    from there on; long rays along a row of boxes and the floor (many candidates, out of their lanes' share)."""
+    b = _floor("row")
+    box = b.shape(scenes.BOX, [0.3, 0.3, 0.3])
+    for i in range(700):
+        b.body(box, scenes.IDENT, np.array([float(i), 0.5, 0.0], np.float32), 1.0)
+    shapes, verts, bodies = scenes.build_records(b.done(dt=1 / 60, iterations=10), jbgpu)
+    ctx = jbgpu.Context()
+    ctx.world_create(shapes, verts, bodies)
+    rng = np.random.default_rng(3)
+    m = 40  # distinct rays: along the whole row (700 candidates), along parts of it, straight down, past everything
+    frm = np.stack([rng.uniform(-5, 705, m), rng.uniform(0.3, 3.0, m), rng.uniform(-0.2, 0.2, m)], 1)
+    to = np.stack([rng.uniform(-5, 705, m), rng.uniform(-1.0, 0.7, m), rng.uniform(-0.2, 0.2, m)], 1)
+    frm[0], to[0] = [-5.0, 0.75, 0.25], [705.0, 0.79, 0.28]  # above every box, inside their margins' AABBs
+    to[1:10, [0, 2]] = frm[1:10, [0, 2]]
+    frm[10], to[10] = [0.0, 50.0, 0.0], [10.0, 60.0, 0.0]
+    frm, to = frm.astype(np.float32), to.astype(np.float32)
+    orc = pyoracle.World(shapes, verts, bodies, iterations=10, order=0)
+    want = orc.ray_test(frm, to)
+    pick = np.arange(n) % m
+    got = ctx.ray_test(frm[pick], to[pick])
+    for g, w in zip(got, want):
+        assert np.array_equal(np.asarray(g).view(np.uint32), np.asarray(w)[pick].view(np.uint32))
+    ctx.close()
