@@ -736,6 +736,55 @@ __global__ __launch_bounds__(kTraverseBlock) void kTraverse(int n, const int* __
   }
 }
 
+// Every pair of a small proxy set, without a tree: a block takes 256 proxies (one per thread) against a chunk of
+// proxies whose boxes its waves read as scalars.  The test is the tree's: same world, candidate boxes, filter words,
+// then the quantised boxes (AxisSweep3; the candidate box is the exact one otherwise).  Pairs are staged in LDS behind
+// one global reservation per block.
+constexpr int kTilePairs = 256;
+constexpr int kTileStage = 2048;
+__global__ __launch_bounds__(kTilePairs) void kPairTiles(int n, int chunk, const float4* __restrict__ cand, int mode,
+                                                         const int* __restrict__ q, int bits,
+                                                         unsigned long long* counter, uint64_t* out, int64_t cap,
+                                                         const int* __restrict__ abortFlag) {
+  const int first = blockIdx.x * kTilePairs;
+  const int j0 = max((int)blockIdx.y * chunk, first + 1), j1 = min(n, ((int)blockIdx.y + 1) * chunk);
+  if (j0 >= j1 || (abortFlag && *abortFlag)) return;  // no pair (i, j) with i < j in this tile
+  __shared__ unsigned int sCount;
+  __shared__ unsigned long long sBase;
+  __shared__ uint64_t sKeys[kTileStage];
+  if (threadIdx.x == 0) sCount = 0;
+  __syncthreads();
+  const int i = first + threadIdx.x;
+  const bool in = i < n;
+  const float4 amn = in ? cand[2 * i] : make_float4(0, 0, 0, 0), amx = in ? cand[2 * i + 1] : make_float4(0, 0, 0, 0);
+  const int wa = __float_as_int(amn.w), fa = __float_as_int(amx.w);
+  auto report = [&](int j, int fb) {
+    if (!in || j <= i || (fa & (fb >> 16) & 0xffff) == 0 || (fb & (fa >> 16) & 0xffff) == 0) return;
+    if (mode == JBGPU_BP_SAP16 || mode == JBGPU_BP_SAP32) {
+      const int* A = q + 6 * i;
+      const int* B = q + 6 * j;
+      for (int ax = 0; ax < 3; ax++)
+        if (A[3 + ax] < B[ax] || B[3 + ax] < A[ax]) return;
+    }
+    const unsigned int slot = atomicAdd(&sCount, 1u);
+    if (slot < (unsigned)kTileStage) sKeys[slot] = ((uint64_t)(i + 1) << bits) | (uint64_t)(j + 1);
+    else emit(i, j, bits, counter, out, cap);
+  };
+#pragma unroll 4
+  for (int j = j0; j < j1; j++) {
+    const float4 bmn = cand[2 * j], bmx = cand[2 * j + 1];
+    const bool meet = (amn.x <= bmx.x) & (amx.x >= bmn.x) & (amn.y <= bmx.y) & (amx.y >= bmn.y) & (amn.z <= bmx.z) &
+                      (amx.z >= bmn.z) & (wa == __float_as_int(bmn.w));
+    if (meet) report(j, __float_as_int(bmx.w));
+  }
+  __syncthreads();
+  const unsigned int staged = min(sCount, (unsigned int)kTileStage);
+  if (threadIdx.x == 0) sBase = staged ? atomicAdd(counter, (unsigned long long)staged) : 0ull;
+  __syncthreads();
+  for (unsigned int k = threadIdx.x; k < staged; k += kTilePairs)
+    if ((int64_t)(sBase + k) < cap) out[sBase + k] = sKeys[k];
+}
+
 // per world w: range[2w], range[2w + 1] = its part of the huge list (sorted by world, then index); the
 // table is cleared to empty ranges beforehand
 __global__ void kHugeRanges(int nh, const int* __restrict__ dn, const int* __restrict__ hugeWorld, int* range) {
@@ -1142,6 +1191,23 @@ void rayBuildTree(Ctx& c) {
   }
 }
 
+// Proxy sets up to this size are tested pair by pair: one launch and no host wait where the tree takes about 24 launches
+// and reads the huge-proxy count back, and no long dependent walk.  Whole calls, tree / pair by pair: setAabb and pairs
+// of scattered boxes 5000 250 / 107 us, 20,011 270 / 225, 25,000 270 / 267, 30,000 270 / 333; a step of 28 bodies
+// 690 / 545 us, 1001 1030 / 759, of piles of 3000 2580 / 2250, 24,000 2260 / 2000, 32,000 2390 / 2230, 40,000 2590 / 2520.
+constexpr int kPairByPair = 96 * kTilePairs;
+static bool pairByPair(const Ctx& c) {
+  return c.np <= kPairByPair && c.blockSize == 0;  // the block-partitioned sweeps need the tree's order
+}
+static void launchPairTiles(Ctx& c, int bits, const int* abortFlag) {
+  const int n = c.np, tiles = gridFor(n, kTilePairs);
+  // chunks of 32 proxies for the smallest sets, so that they spread over the chip, up to 256 for the largest
+  const int chunk = (int)std::min<int64_t>(256, std::max<int64_t>(32, ((int64_t)n * tiles / 1024 + 3) / 4 * 4));
+  hipLaunchKernelGGL(kPairTiles, dim3(tiles, gridFor(n, chunk)), dim3(kTilePairs), 0, c.stream, n, chunk,
+                     (const float4*)c.cand.p, c.bpMode, (const int*)c.q.p, bits, c.counter.p, c.rawKeys.p, c.pairCap,
+                     abortFlag);
+}
+
 void bpFindPairs(Ctx& c) {
   const int n = c.np;
   const int bits = bitsFor((int64_t)n + 1);
@@ -1158,83 +1224,91 @@ void bpFindPairs(Ctx& c) {
     c.stageCurrent = P.newStage;
   }
   c.rotationPending = false;
-  JB_CHECK(hipMemsetAsync(c.counter.p, 0, 8 * sizeof(unsigned long long), s));
-  // centre bounds and extent statistics (two-stage reduction)
-  tBegin(c, T_BVH);
-  unsigned int* bounds = (unsigned int*)c.bounds.p;
-  float* stats = c.bounds.p + 8;
-  unsigned int* part = (unsigned int*)c.bounds.p + 16;
-  const int nparts = std::min(gridFor(n), kStatBlocks);
-  hipLaunchKernelGGL(kProxyStats, dim3(nparts), dim3(256), 0, s, n, (const float*)c.cand.p, (const int*)c.isHuge.p,
-                     part);
-  hipLaunchKernelGGL(kProxyStatsFinal, dim3(1), dim3(256), 0, s, nparts, (const unsigned int*)part, bounds, stats);
-  // huge proxies (absolutely or relatively large), listed in index order
-  hipLaunchKernelGGL(kCountLarge, dim3(gridFor(n)), dim3(256), 0, s, n, kLargeFactor, (const float*)c.cand.p,
-                     stats, (const int*)c.isHuge.p);
-  hipLaunchKernelGGL(kMarkLarge, dim3(gridFor(n)), dim3(256), 0, s, n, kLargeFactor, kLargeCap,
-                     (const float*)c.cand.p, (const float*)stats, c.isHuge.p);
-  int* hugeCount = (int*)(c.counter.p + 1);
-  primSelectIndex(c, (const int*)c.isHuge.p, n, c.hugeList.p, hugeCount);
-  // Morton codes
-  const MortonOrder mo = mortonOrder(c, s, n, c.cand.p, c.isHuge.p, (const unsigned int*)bounds, c.morton.p,
-                                     c.mortonAlt.p, c.order.p, c.orderAlt.p);
-  int hcount = 0;
-  JB_CHECK(hipMemcpyAsync(&hcount, hugeCount, sizeof(hcount), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipStreamSynchronize(s));
-  c.nHuge = hcount;
-  c.st.huge = c.nHuge;
-  const int* order = mo.order;
-  c.sortedOrder = order;
-  const int nn = n - c.nHuge;  // leaves in the tree
-  if (c.nHuge > 0) {  // per-world lookup: the index-ordered list sorted stably by world, i.e. by (world, index)
-    hipLaunchKernelGGL(kHugeWorlds, dim3(gridFor(c.nHuge)), dim3(256), 0, s, c.nHuge, (const int*)nullptr, (int*)nullptr, (const int*)c.hugeList.p,
-                       (const int*)c.world.p, c.hugeWorld.p);
-    if (c.worldBits > 0) {
-      Db<int> hk(c.hugeWorld.p, c.hugeWorldAlt.p);
-      Db<int> hv(c.hugeList.p, c.hugeListAlt.p);
-      primSortPairs(c, hk, hv, c.nHuge, 0, c.worldBits);
-      if (hk.Current() != c.hugeWorld.p)
-        JB_CHECK(hipMemcpyAsync(c.hugeWorld.p, hk.Current(), c.nHuge * sizeof(int), hipMemcpyDeviceToDevice, s));
-      if (hv.Current() != c.hugeList.p)
-        JB_CHECK(hipMemcpyAsync(c.hugeList.p, hv.Current(), c.nHuge * sizeof(int), hipMemcpyDeviceToDevice, s));
+  const bool tiles = pairByPair(c);
+  const int* order = nullptr;
+  int nn = 0;  // leaves in the tree
+  c.nHuge = 0;
+  c.sortedOrder = nullptr;
+  if (!tiles) {
+    JB_CHECK(hipMemsetAsync(c.counter.p, 0, 8 * sizeof(unsigned long long), s));
+    // centre bounds and extent statistics (two-stage reduction)
+    tBegin(c, T_BVH);
+    unsigned int* bounds = (unsigned int*)c.bounds.p;
+    float* stats = c.bounds.p + 8;
+    unsigned int* part = (unsigned int*)c.bounds.p + 16;
+    const int nparts = std::min(gridFor(n), kStatBlocks);
+    hipLaunchKernelGGL(kProxyStats, dim3(nparts), dim3(256), 0, s, n, (const float*)c.cand.p, (const int*)c.isHuge.p,
+                       part);
+    hipLaunchKernelGGL(kProxyStatsFinal, dim3(1), dim3(256), 0, s, nparts, (const unsigned int*)part, bounds, stats);
+    // huge proxies (absolutely or relatively large), listed in index order
+    hipLaunchKernelGGL(kCountLarge, dim3(gridFor(n)), dim3(256), 0, s, n, kLargeFactor, (const float*)c.cand.p,
+                       stats, (const int*)c.isHuge.p);
+    hipLaunchKernelGGL(kMarkLarge, dim3(gridFor(n)), dim3(256), 0, s, n, kLargeFactor, kLargeCap,
+                       (const float*)c.cand.p, (const float*)stats, c.isHuge.p);
+    int* hugeCount = (int*)(c.counter.p + 1);
+    primSelectIndex(c, (const int*)c.isHuge.p, n, c.hugeList.p, hugeCount);
+    // Morton codes
+    const MortonOrder mo = mortonOrder(c, s, n, c.cand.p, c.isHuge.p, (const unsigned int*)bounds, c.morton.p,
+                                       c.mortonAlt.p, c.order.p, c.orderAlt.p);
+    int hcount = 0;
+    JB_CHECK(hipMemcpyAsync(&hcount, hugeCount, sizeof(hcount), hipMemcpyDeviceToHost, s));
+    JB_CHECK(hipStreamSynchronize(s));
+    c.nHuge = hcount;
+    order = mo.order;
+    c.sortedOrder = order;
+    nn = n - c.nHuge;
+    if (c.nHuge > 0) {  // per-world lookup: the index-ordered list sorted stably by world, i.e. by (world, index)
+      hipLaunchKernelGGL(kHugeWorlds, dim3(gridFor(c.nHuge)), dim3(256), 0, s, c.nHuge, (const int*)nullptr, (int*)nullptr, (const int*)c.hugeList.p,
+                         (const int*)c.world.p, c.hugeWorld.p);
+      if (c.worldBits > 0) {
+        Db<int> hk(c.hugeWorld.p, c.hugeWorldAlt.p);
+        Db<int> hv(c.hugeList.p, c.hugeListAlt.p);
+        primSortPairs(c, hk, hv, c.nHuge, 0, c.worldBits);
+        if (hk.Current() != c.hugeWorld.p)
+          JB_CHECK(hipMemcpyAsync(c.hugeWorld.p, hk.Current(), c.nHuge * sizeof(int), hipMemcpyDeviceToDevice, s));
+        if (hv.Current() != c.hugeList.p)
+          JB_CHECK(hipMemcpyAsync(c.hugeList.p, hv.Current(), c.nHuge * sizeof(int), hipMemcpyDeviceToDevice, s));
+      }
     }
+    if (c.nHuge > 0) {
+      c.hugeRange.ensure(2 * ((size_t)c.maxWorld + 1));
+      JB_CHECK(hipMemsetAsync(c.hugeRange.p, 0, 2 * ((size_t)c.maxWorld + 1) * sizeof(int), s));
+      hipLaunchKernelGGL(kHugeRanges, dim3(gridFor(c.nHuge)), dim3(256), 0, s, c.nHuge, (const int*)nullptr, (const int*)c.hugeWorld.p,
+                         c.hugeRange.p);
+    }
+    if (nn >= 2) {
+      hipLaunchKernelGGL(kGatherLeaves<true>, dim3(gridFor(nn)), dim3(256), 0, s, nn, (const int*)nullptr, order, c.cand.p, c.world.p,
+                         c.leafBox.p, c.bpMode, (const float*)c.aabb.p, (const int*)c.q.p, (const int*)c.filt.p,
+                         (int4*)c.leafExact.p);
+      launchBuild(s, gridFor(nn - 1), nn, nullptr, mo, c.nodeChild.p, c.nodeFirst.p, c.nodeLast.p);
+      const int n1 = (nn + 31) / 32, n2 = (n1 + 31) / 32, n3 = (n2 + 31) / 32;
+      float* c1 = c.chunkBox.p;
+      float* c2 = c1 + 8 * (size_t)n1;
+      float* c3 = c2 + 8 * (size_t)n2;
+      hipLaunchKernelGGL(kChunk, dim3(gridFor(nn)), dim3(256), 0, s, nn, (const int*)nullptr, c.leafBox.p, c1);
+      hipLaunchKernelGGL(kChunk, dim3(gridFor(n1)), dim3(256), 0, s, n1, (const int*)nullptr, c1, c2);
+      hipLaunchKernelGGL(kChunk, dim3(gridFor(n2)), dim3(256), 0, s, n2, (const int*)nullptr, c2, c3);
+      (void)n3;
+      hipLaunchKernelGGL(kNodeBoxes, dim3(gridFor(nn - 1)), dim3(256), 0, s, nn, (const int*)nullptr, c.nodeFirst.p, c.nodeLast.p,
+                         c.leafBox.p, c1, c2, c3, c.nodeBox.p);
+      hipLaunchKernelGGL(kNodeRecords, dim3(gridFor(nn - 1)), dim3(256), 0, s, nn, (const int*)nullptr, (const int*)c.nodeChild.p,
+                         (const int*)c.nodeLast.p, (const float*)c.leafBox.p, (const float*)c.nodeBox.p,
+                         (float4*)c.nodeRec.p);
+      if (wide)
+        hipLaunchKernelGGL(kNodeRecords4, dim3(gridFor(nn - 1)), dim3(256), 0, s, nn, (const int*)nullptr, (const float4*)c.nodeRec.p,
+                           (float4*)c.nodeRec4.p);
+    }
+    tEnd(c, T_BVH);
   }
-  if (c.nHuge > 0) {
-    c.hugeRange.ensure(2 * ((size_t)c.maxWorld + 1));
-    JB_CHECK(hipMemsetAsync(c.hugeRange.p, 0, 2 * ((size_t)c.maxWorld + 1) * sizeof(int), s));
-    hipLaunchKernelGGL(kHugeRanges, dim3(gridFor(c.nHuge)), dim3(256), 0, s, c.nHuge, (const int*)nullptr, (const int*)c.hugeWorld.p,
-                       c.hugeRange.p);
-  }
-  if (nn >= 2) {
-    hipLaunchKernelGGL(kGatherLeaves<true>, dim3(gridFor(nn)), dim3(256), 0, s, nn, (const int*)nullptr, order, c.cand.p, c.world.p,
-                       c.leafBox.p, c.bpMode, (const float*)c.aabb.p, (const int*)c.q.p, (const int*)c.filt.p,
-                       (int4*)c.leafExact.p);
-    launchBuild(s, gridFor(nn - 1), nn, nullptr, mo, c.nodeChild.p, c.nodeFirst.p, c.nodeLast.p);
-    const int n1 = (nn + 31) / 32, n2 = (n1 + 31) / 32, n3 = (n2 + 31) / 32;
-    float* c1 = c.chunkBox.p;
-    float* c2 = c1 + 8 * (size_t)n1;
-    float* c3 = c2 + 8 * (size_t)n2;
-    hipLaunchKernelGGL(kChunk, dim3(gridFor(nn)), dim3(256), 0, s, nn, (const int*)nullptr, c.leafBox.p, c1);
-    hipLaunchKernelGGL(kChunk, dim3(gridFor(n1)), dim3(256), 0, s, n1, (const int*)nullptr, c1, c2);
-    hipLaunchKernelGGL(kChunk, dim3(gridFor(n2)), dim3(256), 0, s, n2, (const int*)nullptr, c2, c3);
-    (void)n3;
-    hipLaunchKernelGGL(kNodeBoxes, dim3(gridFor(nn - 1)), dim3(256), 0, s, nn, (const int*)nullptr, c.nodeFirst.p, c.nodeLast.p,
-                       c.leafBox.p, c1, c2, c3, c.nodeBox.p);
-    hipLaunchKernelGGL(kNodeRecords, dim3(gridFor(nn - 1)), dim3(256), 0, s, nn, (const int*)nullptr, (const int*)c.nodeChild.p,
-                       (const int*)c.nodeLast.p, (const float*)c.leafBox.p, (const float*)c.nodeBox.p,
-                       (float4*)c.nodeRec.p);
-    if (wide)
-      hipLaunchKernelGGL(kNodeRecords4, dim3(gridFor(nn - 1)), dim3(256), 0, s, nn, (const int*)nullptr, (const float4*)c.nodeRec.p,
-                         (float4*)c.nodeRec4.p);
-  }
-  tEnd(c, T_BVH);
+  c.st.huge = c.nHuge;
   PairTest T{c.bpMode, c.aabb.p, c.q.p, c.filt.p, c.world.p};
   for (int attempt = 0; attempt < 3; attempt++) {
     if (c.pairCap < 1024) c.pairCap = std::max<int64_t>(1024, 8 * (int64_t)n);
     c.rawKeys.ensure(c.pairCap);
     c.rawKeysAlt.ensure(c.pairCap);
-    JB_CHECK(hipMemsetAsync(c.counter.p, 0, 2 * sizeof(unsigned long long), s));
+    JB_CHECK(hipMemsetAsync(c.counter.p, 0, (tiles ? 8 : 2) * sizeof(unsigned long long), s));
     if (attempt == 0) tBegin(c, T_TRAVERSE);
+    if (tiles) launchPairTiles(c, bits, nullptr);
     if (nn >= 2)
       hipLaunchKernelGGL(wide ? kTraverse<4> : kTraverse<2>, dim3(gridFor(nn, kTraverseBlock)), dim3(kTraverseBlock),
                          0, s, nn, (const int*)nullptr, order, c.leafBox.p, (const float4*)(wide ? c.nodeRec4.p : c.nodeRec.p),
@@ -1245,7 +1319,8 @@ void bpFindPairs(Ctx& c) {
       hipLaunchKernelGGL(kHuge, dim3(gridFor(n, kHugeBlock)), dim3(kHugeBlock), 0, s, n, (const int*)c.hugeRange.p,
                          (const int*)c.hugeList.p, c.isHuge.p, c.cand.p, T, bits, c.counter.p, c.rawKeys.p,
                          c.pairCap);
-    unsigned long long cnt[3] = {0, 0, 0};
+    c.counterHost.ensure(8);
+    unsigned long long* cnt = c.counterHost.p;
     JB_CHECK(hipMemcpyAsync(cnt, c.counter.p, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     JB_CHECK(hipStreamSynchronize(s));
     if (cnt[2]) throw std::runtime_error("broadphase traversal stack overflow");
@@ -1461,6 +1536,17 @@ const uint64_t* bpStepGraph(Ctx& c) {
                      (const int*)c.filt.p, (const int*)(gc + kGcAbort));
   c.stageCurrent = P.newStage;
   c.rotationPending = false;
+  auto foundAndSorted = [&]() {
+    hipLaunchKernelGGL(kGraphPairsFound, dim3(1), dim3(1), 0, s, (const unsigned long long*)c.counter.p, c.pairCap, gc);
+    Db<uint64_t> kk(c.rawKeys.p, c.rawKeysAlt.p);
+    primSortKeysDev(c, kk, (const int*)(gc + kGcPairs), (int)c.pairCap, 0, 2 * bits);
+    return (const uint64_t*)kk.Current();
+  };
+  if (pairByPair(c)) {
+    c.sortedOrder = nullptr;
+    launchPairTiles(c, bits, gc + kGcAbort);
+    return foundAndSorted();
+  }
   unsigned int* bounds = (unsigned int*)c.bounds.p;
   float* stats = c.bounds.p + 8;
   unsigned int* part = (unsigned int*)c.bounds.p + 16;
@@ -1513,10 +1599,7 @@ const uint64_t* bpStepGraph(Ctx& c) {
                      (int*)(c.counter.p + 2), c.pairStage.p);
   hipLaunchKernelGGL(kHuge, dim3(gridFor(n, kHugeBlock)), dim3(kHugeBlock), 0, s, n, (const int*)c.hugeRange.p,
                      (const int*)hv.Current(), c.isHuge.p, c.cand.p, T, bits, c.counter.p, c.rawKeys.p, c.pairCap);
-  hipLaunchKernelGGL(kGraphPairsFound, dim3(1), dim3(1), 0, s, (const unsigned long long*)c.counter.p, c.pairCap, gc);
-  Db<uint64_t> kk(c.rawKeys.p, c.rawKeysAlt.p);
-  primSortKeysDev(c, kk, (const int*)(gc + kGcPairs), (int)c.pairCap, 0, 2 * bits);
-  return kk.Current();
+  return foundAndSorted();
 }
 
 void bpRemapGraph(Ctx& c, const uint64_t* sorted) {

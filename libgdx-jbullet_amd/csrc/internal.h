@@ -266,6 +266,7 @@ struct Ctx {
   DBuf<uint64_t> rawKeys, rawKeysAlt;
   DBuf<uint64_t> pairStage;  // per traversal block: staged pair keys
   DBuf<unsigned long long> counter;  // misc device counters
+  HBuf<unsigned long long> counterHost;  // their readback
   DBuf<int> primTmp;  // scratch of the device-wide scans, compactions and sorts (prim.hip)
   HBuf<int> primErrHost;  // the sorts' error word, read back after a step
   int64_t pairCap = 0;

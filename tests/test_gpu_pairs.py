@@ -1,0 +1,74 @@
+"""GPU parity of the pair search where it changes form: small proxy sets are tested pair by pair (256 proxies against a
+chunk at a time), larger ones through the tree; pair sets bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+import jbgpu
+import pyoracle
+from test_gpu_parity import MODES, WMAX, WMIN
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(mode, boxes, group, mask, world):
+    ctx = jbgpu.Context(bp_mode=MODES[mode], world_min=WMIN, world_max=WMAX)
+    ctx.bp_create_proxies(boxes, group, mask, world)
+    orc = pyoracle.Broadphase(MODES[mode], np.array(WMIN, np.float32), np.array(WMAX, np.float32))
+    orc.create(boxes, group, mask)
+    if world is not None:
+        orc.set_worlds(world)
+    return ctx, orc
+
+
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 2049])
+def test_pair_by_pair_tile_edges(mode, n):
+    """Both sides of a tile and a chunk, with filters, worlds, boxes that touch exactly, coincident boxes and one box
+    around everything."""
+    rng = np.random.default_rng(n)
+    side = 3.0 * n ** (1.0 / 3.0)
+    c = rng.integers(0, max(2, int(side)), (n, 3)).astype(np.float32)  # on a grid: faces touch, some boxes coincide
+    h = rng.choice(np.array([0.25, 0.5, 1.0], np.float32), (n, 3))
+    v = rng.normal(0, 5, (n, 3)).astype(np.float32)
+    h[n // 2] = 500.0
+    group = rng.integers(1, 4, n).astype(np.int16)
+    mask = rng.integers(0, 4, n).astype(np.int16)
+    mask[rng.random(n) < 0.3] = -1
+    world = rng.integers(0, 3, n).astype(np.int32)
+    ctx, orc = _both(mode, np.concatenate([c - h, c + h], 1), group, mask, world)
+    for step in range(4):
+        boxes = np.concatenate([c - h, c + h], 1).astype(np.float32)
+        ctx.bp_set_aabbs(boxes)
+        orc.set_all(boxes)
+        ctx.bp_calculate_overlapping_pairs()
+        assert np.array_equal(ctx.bp_pairs(), orc.step()), f"{mode} {n} step {step}"
+        c = (c + v * np.float32(1.0 / 60.0)).astype(np.float32)
+    ctx.close()
+
+
+@pytest.mark.parametrize("mode", ["dbvt", "sap16"])
+@pytest.mark.parametrize("n", [24576, 24577])
+def test_both_sides_of_the_tree_limit(mode, n):
+    rng = np.random.default_rng(7)
+    c = rng.uniform(0, 250, (n, 3)).astype(np.float32)
+    h = rng.lognormal(0.0, 0.7, (n, 3)).astype(np.float32)
+    boxes = np.concatenate([c - h, c + h], 1).astype(np.float32)
+    ctx, orc = _both(mode, boxes, None, None, None)
+    for step in range(2):
+        ctx.bp_set_aabbs(boxes)
+        orc.set_all(boxes)
+        ctx.bp_calculate_overlapping_pairs()
+        assert np.array_equal(ctx.bp_pairs(), orc.step(cap=1 << 21)), f"{mode} {n} step {step}"
+    ctx.close()
+
+
+def test_dense_tiles_past_their_staging():
+    """Every box overlaps every other: a tile finds more pairs than its staging holds, and the pair capacity grows."""
+    n = 700
+    boxes = np.tile(np.array([[0, 0, 0, 1, 1, 1]], np.float32), (n, 1))
+    ctx, orc = _both("dbvt", boxes, None, None, None)
+    ctx.bp_set_aabbs(boxes)
+    orc.set_all(boxes)
+    assert ctx.bp_calculate_overlapping_pairs() == n * (n - 1) // 2
+    assert np.array_equal(ctx.bp_pairs(), orc.step(cap=1 << 19))
+    ctx.close()
