@@ -1345,9 +1345,12 @@ void bpFindPairs(Ctx& c) {
 }
 
 // ---- proxy removal and pair deltas ------------------------------------------------------------------
-__global__ void kKillProxies(int n, const int* __restrict__ uids, int* filt) {
+// filter words cleared, also in the candidate records (null: none yet) that the next pair query may read
+__global__ void kKillProxies(int n, const int* __restrict__ uids, int* filt, float* cand) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) filt[uids[i] - 1] = 0;
+  if (i >= n) return;
+  filt[uids[i] - 1] = 0;
+  if (cand) cand[8 * (size_t)(uids[i] - 1) + 7] = __int_as_float(0);
 }
 // 1 for the keys whose proxies both still pair (a destroyed proxy has group and mask 0)
 __global__ void kPairLive(int64_t n, const uint64_t* __restrict__ keys, const int* __restrict__ filt, int* flag) {
@@ -1401,7 +1404,8 @@ void bpDestroyProxies(Ctx& c, int n, const int32_t* uids) {
   c.counter.ensure(8);
   c.deltaFlag.ensure(n);
   JB_CHECK(hipMemcpyAsync(c.deltaFlag.p, u.data(), n * sizeof(int), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(kKillProxies, dim3(gridFor(n)), dim3(256), 0, s, n, (const int*)c.deltaFlag.p, c.filt.p);
+  hipLaunchKernelGGL(kKillProxies, dim3(gridFor(n)), dim3(256), 0, s, n, (const int*)c.deltaFlag.p, c.filt.p,
+                     c.cand.n >= 8 * (size_t)c.np ? c.cand.p : nullptr);
   // removeOverlappingPairsContainingProxy: the pairs leave the current set and the previous one (so
   // the next delta lists them in neither direction)
   const int64_t sizes[2] = {c.npairs, c.npairsOld};

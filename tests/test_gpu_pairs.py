@@ -72,3 +72,23 @@ def test_dense_tiles_past_their_staging():
     assert ctx.bp_calculate_overlapping_pairs() == n * (n - 1) // 2
     assert np.array_equal(ctx.bp_pairs(), orc.step(cap=1 << 19))
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [300, 30000])
+def test_proxies_destroyed_between_set_aabb_and_the_query(n):
+    """destroyProxy after setAabb and before the pair query: the destroyed proxies pair no more."""
+    rng = np.random.default_rng(4)
+    c = rng.uniform(0, 3.0 * n ** (1.0 / 3.0), (n, 3)).astype(np.float32)
+    boxes = np.concatenate([c - 1, c + 1], 1).astype(np.float32)
+    ctx, orc = _both("dbvt", boxes, None, None, None)
+    ctx.bp_set_aabbs(boxes)
+    orc.set_all(boxes)
+    dead = rng.choice(n, n // 5, replace=False) + 1
+    ctx.bp_destroy_proxies(dead)
+    orc.destroy(dead)
+    ctx.bp_calculate_overlapping_pairs()
+    got = ctx.bp_pairs()
+    lo, hi = (got >> np.uint64(32)).astype(np.int64), (got & np.uint64(0xffffffff)).astype(np.int64)
+    assert len(got) and not (np.isin(lo, dead) | np.isin(hi, dead)).any()
+    assert np.array_equal(got, orc.step())
+    ctx.close()
