@@ -345,6 +345,10 @@ struct Ctx {
   DBuf<int> flowCtl;
   HBuf<int> flowErrHost;
   bool oddBodies = false;  // a body flagged static has a mass
+  // slot order of a small step: its counts and colour starts, and the last step's manifolds
+  DBuf<int> smallInfo;
+  HBuf<int> smallInfoHost;
+  int64_t smallTooMany = 0;
   DBuf<int2> activeBodies;   // per active manifold: body A, body B
   DBuf<int> colorStart;
   HBuf<int> batchHost;  // readback of the colour batches: count, first slots, boundary flags

@@ -148,3 +148,40 @@ def test_ray_counts_around_the_lane_split(n):
     for g, w in zip(got, want):
         assert np.array_equal(np.asarray(g).view(np.uint32), np.asarray(w)[pick].view(np.uint32))
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [1023, 1025, 5119, 5120])
+def test_small_step_limits(n):
+    """n boxes at rest and the floor on both sides of a thousand manifolds and of the bodies the one-launch solve order
+    holds (5120 with the floor)."""
+    ctx, orc = _world_pair(_separate(n))
+    for step in range(2):
+        _sync_and_step(ctx, orc)
+        _compare_world(ctx, orc, f"separate {n} step {step}")
+    assert ctx.stats()["manifolds"] == n
+    ctx.close()
+
+
+def test_more_manifolds_than_the_small_order_holds():
+    """4400 boxes stacked two and two on a row of plates: over 8192 manifolds among few bodies, then fewer again."""
+    b = _floor("stacks")
+    box = b.shape(scenes.BOX, [0.5, 0.5, 0.5])
+    side = 16
+    for k in range(side * side * 17):  # a close-packed block: about three manifolds a box
+        x, z, y = k % side, (k // side) % side, k // (side * side)
+        b.body(box, scenes.IDENT, np.array([0.999 * x, 0.499 + 0.998 * y, 0.999 * z], np.float32), 1.0)
+    ctx, orc = _world_pair(b.done(dt=1 / 60, iterations=4), iterations=4)
+    seen = 0
+    for step in range(2):
+        _sync_and_step(ctx, orc)
+        _compare_world(ctx, orc, f"stacks step {step}")
+        seen = max(seen, ctx.stats()["manifolds"])
+    assert seen > 8192
+    bodies = ctx.bodies()
+    bodies[2000:, 9] += 5.0 * np.arange(len(bodies) - 2000)  # most of them flung apart
+    ctx.set_bodies(bodies)
+    for step in range(2):
+        _sync_and_step(ctx, orc)
+        _compare_world(ctx, orc, f"stacks apart step {step}")
+    assert ctx.stats()["manifolds"] <= 8192
+    ctx.close()
