@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "../../include/jbgpu_format.h"
+#include "xfer.h"
 
 namespace jbg {
 
@@ -194,6 +195,7 @@ struct Ctx {
   hipStream_t stream = nullptr;
   int device = 0;  // the HIP device current when the context was created
   std::string err;
+  HostCopy host;  // copies from and to the caller's memory
   // configuration
   int bpMode = JBGPU_BP_DBVT;
   float wmin[3] = {-1000, -1000, -1000}, wmax[3] = {1000, 1000, 1000};
@@ -361,7 +363,7 @@ struct Ctx {
   DBuf<float> mlpNorm;       // input / output normalisation
   DBuf<float> mlpX, mlpY;    // inference / training samples
   DBuf<int> mlpIdx;          // training permutation
-  DBuf<float> mlpG, mlpM, mlpV, mlpLoss;  // gradient, Adam moments, loss accumulator
+  DBuf<float> mlpG, mlpM, mlpV;  // gradient with the loss behind it, Adam moments
   DBuf<uint16_t> mlpFrag;    // per training tile: activations and gradients, fragment-ready
   DBuf<int> mActive;  // active manifold list
   DBuf<int> island;      // island parent forest (root = smallest body index of the island)

@@ -392,7 +392,7 @@ __global__ __launch_bounds__(64) void kMlpFwdBwd(int64_t nb, const int* __restri
   for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const int64_t r = t * 16 + (lane & 15);
     const bool ok = r < nb;
-    const int64_t s = ok ? idx[r] : 0;
+    const int64_t s = !ok ? 0 : idx ? idx[r] : r;
     Acts a;
     f32x4 y = forward<true>(P, W, inputFrag(X + 16 * s, ok, norm, lane), lane, &a);
     // dL/dy' for the mean squared error over nb x 3 normalised outputs
@@ -546,14 +546,13 @@ void mlpInfer(Ctx& c, const float* x, int64_t n, float* y) {
   hipStream_t s = c.stream;
   c.mlpX.ensure((size_t)16 * n);
   c.mlpY.ensure((size_t)3 * n);
-  JB_CHECK(hipMemcpyAsync(c.mlpX.p, x, 16 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
+  c.host.send(s, c.mlpX.p, x, 16 * (size_t)n * sizeof(float));
   tBegin(c, T_MLP);
   hipLaunchKernelGGL(kMlpInfer<false>, dim3(inferGrid(n)), dim3(256), 0, s, n, c.mlpX.p, c.mlpWb.p, c.mlpW.p, c.mlpNorm.p,
                      c.mlpY.p, nullptr, nullptr, nullptr);
   JB_CHECK(hipGetLastError());
   tEnd(c, T_MLP);
-  JB_CHECK(hipMemcpyAsync(y, c.mlpY.p, 3 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipStreamSynchronize(s));
+  c.host.fetch(s, y, c.mlpY.p, 3 * (size_t)n * sizeof(float));
   if (c.timing) tCollect(c);  // outside a step: the kernel's timing region is read here
 }
 
@@ -604,15 +603,17 @@ void mlpInferStatic(Ctx& c, const float* x, int64_t n, float* y) {
 }
 
 namespace {
-// gradient of the loss for the nb samples listed at idx, accumulated into c.mlpG (zeroed here)
-void gradBatch(Ctx& c, const int* idx, int64_t nb, float gscale) {
+// gradient of the loss for the nb samples listed at idx (the first nb without a list), accumulated into c.mlpG (zeroed
+// here); the summed squared error is added to the word behind it, which starts at zero if newLoss
+void gradBatch(Ctx& c, const int* idx, int64_t nb, float gscale, bool newLoss) {
   hipStream_t s = c.stream;
   const int64_t ntiles = (nb + 15) / 16;
   c.mlpFrag.ensure((size_t)ntiles * kTileFrags * 256);
-  hipLaunchKernelGGL(kFillF, dim3(gridFor(kMlpParams)), dim3(256), 0, s, c.mlpG.p, kMlpParams, 0.0f);
+  const int nfill = kMlpParams + (newLoss ? 1 : 0);
+  hipLaunchKernelGGL(kFillF, dim3(gridFor(nfill)), dim3(256), 0, s, c.mlpG.p, nfill, 0.0f);
   const int fb = (int)std::min<int64_t>(ntiles, 8192);
   hipLaunchKernelGGL(kMlpFwdBwd, dim3(fb), dim3(64), 0, s, nb, idx, c.mlpX.p, c.mlpY.p, c.mlpNorm.p, c.mlpWb.p,
-                     c.mlpW.p, c.mlpFrag.p, c.mlpLoss.p, gscale);
+                     c.mlpW.p, c.mlpFrag.p, c.mlpG.p + kMlpParams, gscale);
   const int chunk = 32;
   const int64_t nchunks = (ntiles + chunk - 1) / chunk;
   hipLaunchKernelGGL(kMlpWgrad, dim3((unsigned)(40 * nchunks)), dim3(64), 0, s, ntiles, chunk, c.mlpFrag.p, c.mlpG.p);
@@ -623,11 +624,9 @@ void uploadData(Ctx& c, const float* x, const float* y, int64_t n) {
   hipStream_t s = c.stream;
   c.mlpX.ensure((size_t)16 * n);
   c.mlpY.ensure((size_t)3 * n);
-  c.mlpIdx.ensure((size_t)n);
-  c.mlpG.ensure(kMlpParams);
-  c.mlpLoss.ensure(1);
-  JB_CHECK(hipMemcpyAsync(c.mlpX.p, x, 16 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
-  JB_CHECK(hipMemcpyAsync(c.mlpY.p, y, 3 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
+  c.mlpG.ensure(kMlpParams + 1);
+  c.host.send(s, c.mlpX.p, x, 16 * (size_t)n * sizeof(float));
+  c.host.send(s, c.mlpY.p, y, 3 * (size_t)n * sizeof(float));
 }
 }  // namespace
 
@@ -637,16 +636,11 @@ void mlpGrad(Ctx& c, const float* x, const float* y, int64_t n, float* grad, flo
   if (n > (int64_t)1 << 30) throw std::length_error("too many samples");
   hipStream_t s = c.stream;
   uploadData(c, x, y, n);
-  std::vector<int> idx(n);
-  for (int64_t i = 0; i < n; i++) idx[i] = (int)i;
-  JB_CHECK(hipMemcpyAsync(c.mlpIdx.p, idx.data(), n * sizeof(int), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(kFillF, dim3(1), dim3(64), 0, s, c.mlpLoss.p, 1, 0.0f);
-  gradBatch(c, c.mlpIdx.p, n, 2.0f / (3.0f * (float)n));
-  float l = 0;
-  JB_CHECK(hipMemcpyAsync(grad, c.mlpG.p, kMlpParams * sizeof(float), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(&l, c.mlpLoss.p, sizeof(float), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipStreamSynchronize(s));
-  if (loss) *loss = l / (3.0f * (float)n);
+  gradBatch(c, nullptr, n, 2.0f / (3.0f * (float)n), true);
+  float out[kMlpParams + 1];
+  c.host.fetch(s, out, c.mlpG.p, sizeof(out));
+  std::copy(out, out + kMlpParams, grad);
+  if (loss) *loss = out[kMlpParams] / (3.0f * (float)n);
 }
 
 void mlpTrain(Ctx& c, const float* x, const float* y, int64_t n, int epochs, int batch, float lr, uint64_t seed,
@@ -688,6 +682,7 @@ void mlpTrain(Ctx& c, const float* x, const float* y, int64_t n, int epochs, int
   for (int i = 0; i < kMlpOut * kMlpHid; i++) W[kMlpW4 + i] *= 0.1f;
   mlpSetParams(c, W.data(), norm.data());
   uploadData(c, x, y, n);
+  c.mlpIdx.ensure((size_t)n);
   c.mlpM.ensure(kMlpParams);
   c.mlpV.ensure(kMlpParams);
   hipLaunchKernelGGL(kFillF, dim3(gridFor(kMlpParams)), dim3(256), 0, s, c.mlpM.p, kMlpParams, 0.0f);
@@ -698,11 +693,10 @@ void mlpTrain(Ctx& c, const float* x, const float* y, int64_t n, int epochs, int
   for (int e = 0; e < epochs; e++) {
     std::shuffle(perm.begin(), perm.end(), rng);
     JB_CHECK(hipMemcpyAsync(c.mlpIdx.p, perm.data(), n * sizeof(int), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(kFillF, dim3(1), dim3(64), 0, s, c.mlpLoss.p, 1, 0.0f);
     for (int64_t b0 = 0; b0 < n; b0 += batch) {
       const int64_t nb = std::min<int64_t>(batch, n - b0);
       // the batch is the window [b0, b0 + nb) of the permutation
-      gradBatch(c, c.mlpIdx.p + b0, nb, 2.0f / (3.0f * (float)nb));
+      gradBatch(c, c.mlpIdx.p + b0, nb, 2.0f / (3.0f * (float)nb), b0 == 0);
       step++;
       const float bc1 = 1.0f - std::pow(0.9f, (float)step), bc2 = 1.0f - std::pow(0.999f, (float)step);
       hipLaunchKernelGGL(kMlpAdam, dim3(gridFor(kMlpParams)), dim3(256), 0, s, c.mlpG.p, c.mlpW.p, c.mlpM.p, c.mlpV.p,
@@ -710,7 +704,7 @@ void mlpTrain(Ctx& c, const float* x, const float* y, int64_t n, int epochs, int
       repack(c);
     }
     float l = 0;
-    JB_CHECK(hipMemcpyAsync(&l, c.mlpLoss.p, sizeof(float), hipMemcpyDeviceToHost, s));
+    JB_CHECK(hipMemcpyAsync(&l, c.mlpG.p + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, s));
     JB_CHECK(hipStreamSynchronize(s));
     if (lossPerEpoch) lossPerEpoch[e] = l / (3.0f * (float)n);
   }

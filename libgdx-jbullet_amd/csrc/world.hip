@@ -270,38 +270,37 @@ void bodiesToDevice(Ctx& c, const float* bodies) {
   JB_CHECK(hipStreamSynchronize(s));
 }
 
+// body records (JBGPU_BODY_WORDS words) of bodies first, first + 1, ... from the device's streams, eight threads each
+__global__ void kPackBodies(int first, int n, const float* __restrict__ tr, const float* __restrict__ vel,
+                            const float* __restrict__ props, const float* __restrict__ grav,
+                            const int* __restrict__ act, const float* __restrict__ deact, float4* out) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 8 * n) return;
+  const size_t i = (size_t)first + (t >> 3);
+  const int k = t & 7;
+  const float* T = tr + 12 * i;
+  const float* V = vel + 8 * i;
+  const float* P = props + 8 * i;
+  const float* G = grav + 4 * i;
+  float4 r;
+  if (k < 3) r = ((const float4*)T)[k];
+  else if (k == 3) r = make_float4(V[0], V[1], V[2], V[4]);
+  else if (k == 4) r = make_float4(V[5], V[6], P[0], P[1]);
+  else if (k == 5) r = make_float4(P[2], P[3], G[0], G[1]);
+  else if (k == 6) r = make_float4(G[2], P[4], P[5], P[6]);
+  else r = make_float4(P[7], __int_as_float(act[i]), deact[i], 0.0f);
+  out[t] = r;
+}
+
 void bodiesFromDevice(Ctx& c, float* bodies) {
-  int n = c.nb;
-  std::vector<float> tr(12 * (size_t)n), vel(8 * (size_t)n), props(8 * (size_t)n), grav(4 * (size_t)n), deact(n);
-  std::vector<int> act(n);
-  hipStream_t s = c.stream;
-  JB_CHECK(hipMemcpyAsync(tr.data(), c.tr.p, tr.size() * 4, hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(vel.data(), c.vel.p, vel.size() * 4, hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(props.data(), c.props.p, props.size() * 4, hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(grav.data(), c.grav.p, grav.size() * 4, hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(act.data(), c.act.p, act.size() * 4, hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(deact.data(), c.deact.p, deact.size() * 4, hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipStreamSynchronize(s));
-  for (int i = 0; i < n; i++) {
-    float* r = bodies + (size_t)JBGPU_BODY_WORDS * i;
-    std::memset(r, 0, JBGPU_BODY_WORDS * sizeof(float));
-    for (int k = 0; k < 12; k++) r[k] = tr[12 * i + k];
-    for (int k = 0; k < 3; k++) {
-      r[12 + k] = vel[8 * i + k];
-      r[15 + k] = vel[8 * i + 4 + k];
-      r[22 + k] = grav[4 * i + k];
-    }
-    r[18] = props[8 * i + 0];
-    r[19] = props[8 * i + 1];
-    r[20] = props[8 * i + 2];
-    r[21] = props[8 * i + 3];
-    r[25] = props[8 * i + 4];
-    r[26] = props[8 * i + 5];
-    r[27] = props[8 * i + 6];
-    r[28] = props[8 * i + 7];
-    sti(r + 29, act[i]);
-    r[30] = deact[i];
-  }
+  constexpr size_t kRec = JBGPU_BODY_WORDS * sizeof(float);
+  c.host.fetchWith(c.stream, bodies, (size_t)c.nb * kRec, kRec, [&](void* slot, size_t at, size_t bytes) {
+    const int n = (int)(bytes / kRec);
+    hipLaunchKernelGGL(kPackBodies, dim3(gridFor(8 * (int64_t)n)), dim3(256), 0, c.stream, (int)(at / kRec), n,
+                       (const float*)c.tr.p, (const float*)c.vel.p, (const float*)c.props.p, (const float*)c.grav.p,
+                       (const int*)c.act.p, (const float*)c.deact.p, (float4*)slot);
+    JB_CHECK(hipGetLastError());
+  });
 }
 
 // Host check of caller-supplied pair keys and manifold records before any of them reaches a kernel: keys
@@ -362,9 +361,8 @@ void uploadPairs(Ctx& c, int64_t n, const uint64_t* keys, const float* manifolds
   c.keys[c.cur].ensure(std::max<int64_t>(n, 1));
   c.man[c.cur].ensure((size_t)JBGPU_MANIFOLD_WORDS * std::max<int64_t>(n, 1));
   if (n) {
-    JB_CHECK(hipMemcpy(c.keys[c.cur].p, keys, n * sizeof(uint64_t), hipMemcpyHostToDevice));
-    JB_CHECK(hipMemcpy(c.man[c.cur].p, manifolds, (size_t)n * JBGPU_MANIFOLD_WORDS * sizeof(float),
-                       hipMemcpyHostToDevice));
+    c.host.send(c.stream, c.keys[c.cur].p, keys, n * sizeof(uint64_t));
+    c.host.send(c.stream, c.man[c.cur].p, manifolds, (size_t)n * JBGPU_MANIFOLD_WORDS * sizeof(float));
   }
   c.npairs = n;
   c.npairsOld = 0;
@@ -867,7 +865,7 @@ int jbgpu_bp_set_aabbs(jbgpu_ctx* ctx, int32_t n, const float* aabb6, int32_t on
     const float* d = aabb6;
     if (!on_device) {
       c.candC.ensure(6 * (size_t)n);
-      JB_CHECK(hipMemcpyAsync(c.candC.p, aabb6, 6 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, c.stream));
+      c.host.send(c.stream, c.candC.p, aabb6, 6 * (size_t)n * sizeof(float));
       d = c.candC.p;
     }
     bpUpdateFromAabbs(c, d);
@@ -900,7 +898,7 @@ int jbgpu_bp_get_pairs(jbgpu_ctx* ctx, uint64_t* keys, int64_t cap, int64_t* n) 
     if (!keys) return;
     if (cap < c.npairs) throw std::length_error("pair buffer too small");
     if (c.npairs)
-      JB_CHECK(hipMemcpy(keys, c.keys[c.cur].p, c.npairs * sizeof(uint64_t), hipMemcpyDeviceToHost));
+      c.host.fetch(c.stream, keys, c.keys[c.cur].p, c.npairs * sizeof(uint64_t));
   });
 }
 
@@ -932,15 +930,14 @@ int jbgpu_world_ray_test(jbgpu_ctx* ctx, int32_t n, const float* from3, const fl
     float* dPoint = dNormal + 3 * (size_t)n;
     int* dObj = t.ioInt.p;
     int* dWorld = world ? t.ioInt.p + n : nullptr;
-    JB_CHECK(hipMemcpyAsync(dFrom, from3, 3 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
-    JB_CHECK(hipMemcpyAsync(dTo, to3, 3 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
+    c.host.send(s, dFrom, from3, 3 * (size_t)n * sizeof(float));
+    c.host.send(s, dTo, to3, 3 * (size_t)n * sizeof(float));
     if (world) JB_CHECK(hipMemcpyAsync(dWorld, world, (size_t)n * sizeof(int), hipMemcpyHostToDevice, s));
     rayTest(c, n, dFrom, dTo, group, mask, dWorld, dObj, dFrac, dNormal, dPoint);
-    JB_CHECK(hipMemcpyAsync(obj, dObj, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipMemcpyAsync(fraction, dFrac, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipMemcpyAsync(normal3, dNormal, 3 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipMemcpyAsync(point3, dPoint, 3 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipStreamSynchronize(s));
+    c.host.fetch(s, obj, dObj, (size_t)n * sizeof(int));
+    c.host.fetch(s, fraction, dFrac, (size_t)n * sizeof(float));
+    c.host.fetch(s, normal3, dNormal, 3 * (size_t)n * sizeof(float));
+    c.host.fetch(s, point3, dPoint, 3 * (size_t)n * sizeof(float));
   });
 }
 
@@ -1423,15 +1420,14 @@ int jbgpu_world_convex_sweep_test(jbgpu_ctx* ctx, const float* cast_shape, int32
     float* dPoint = dNormal + 3 * (size_t)n;
     int* dObj = t.ioInt.p;
     int* dWorld = world ? t.ioInt.p + n : nullptr;
-    JB_CHECK(hipMemcpyAsync(dFrom, from12, 12 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
-    JB_CHECK(hipMemcpyAsync(dTo, to12, 12 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, s));
+    c.host.send(s, dFrom, from12, 12 * (size_t)n * sizeof(float));
+    c.host.send(s, dTo, to12, 12 * (size_t)n * sizeof(float));
     if (world) JB_CHECK(hipMemcpyAsync(dWorld, world, (size_t)n * sizeof(int), hipMemcpyHostToDevice, s));
     sweepTest(c, n, cast_shape, dFrom, dTo, group, mask, dWorld, dObj, dFrac, dNormal, dPoint);
-    JB_CHECK(hipMemcpyAsync(obj, dObj, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipMemcpyAsync(fraction, dFrac, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipMemcpyAsync(normal3, dNormal, 3 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipMemcpyAsync(point3, dPoint, 3 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost, s));
-    JB_CHECK(hipStreamSynchronize(s));
+    c.host.fetch(s, obj, dObj, (size_t)n * sizeof(int));
+    c.host.fetch(s, fraction, dFrac, (size_t)n * sizeof(float));
+    c.host.fetch(s, normal3, dNormal, 3 * (size_t)n * sizeof(float));
+    c.host.fetch(s, point3, dPoint, 3 * (size_t)n * sizeof(float));
   });
 }
 
@@ -1459,10 +1455,9 @@ int jbgpu_world_get_pairs(jbgpu_ctx* ctx, uint64_t* keys, float* manifolds) {
   return guard(ctx, [&] {
     Ctx& c = ctx->c;
     if (c.npairs == 0) return;
-    if (keys) JB_CHECK(hipMemcpy(keys, c.keys[c.cur].p, c.npairs * sizeof(uint64_t), hipMemcpyDeviceToHost));
+    if (keys) c.host.fetch(c.stream, keys, c.keys[c.cur].p, c.npairs * sizeof(uint64_t));
     if (manifolds)
-      JB_CHECK(hipMemcpy(manifolds, c.man[c.cur].p, (size_t)c.npairs * JBGPU_MANIFOLD_WORDS * sizeof(float),
-                         hipMemcpyDeviceToHost));
+      c.host.fetch(c.stream, manifolds, c.man[c.cur].p, (size_t)c.npairs * JBGPU_MANIFOLD_WORDS * sizeof(float));
   });
 }
 
@@ -1490,8 +1485,7 @@ int jbgpu_np_dispatch(jbgpu_ctx* ctx, int64_t n, const uint64_t* keys, const flo
     JB_CHECK(hipStreamSynchronize(c.stream));
     npCollectStats(c);
     if (n)
-      JB_CHECK(hipMemcpy(manifolds_out, c.man[c.cur].p, (size_t)n * JBGPU_MANIFOLD_WORDS * sizeof(float),
-                         hipMemcpyDeviceToHost));
+      c.host.fetch(c.stream, manifolds_out, c.man[c.cur].p, (size_t)n * JBGPU_MANIFOLD_WORDS * sizeof(float));
     if (c.epaOverflow)
       throw std::length_error("EPA workspace overflow in this pass (the manifolds have been updated)");
   });
