@@ -164,58 +164,42 @@ struct Sub {
   __device__ void setBC(float a, float b, float c, float d) { bc[0] = a; bc[1] = b; bc[2] = c; bc[3] = d; }
 };
 
-__device__ bool triClosest(V3 p, V3 a, V3 b, V3 c, Sub& r) {
-  r.used = 0;
-  V3 ab = sub(b, a), ac = sub(c, a), ap = sub(p, a);
-  float d1 = dot(ab, ap), d2 = dot(ac, ap);
-  if (d1 <= 0.0f && d2 <= 0.0f) {
-    r.closest = a; r.used = 1; r.setBC(1, 0, 0, 0);
-    return true;
-  }
-  V3 bp = sub(p, b);
-  float d3 = dot(ab, bp), d4 = dot(ac, bp);
-  if (d3 >= 0.0f && d4 <= d3) {
-    r.closest = b; r.used = 2; r.setBC(0, 1, 0, 0);
-    return true;
-  }
-  float vc = d1 * d4 - d3 * d2;
-  if (vc <= 0.0f && d1 >= 0.0f && d3 <= 0.0f) {
-    float v = d1 / (d1 - d3);
-    r.closest = v3(v * ab.x + a.x, v * ab.y + a.y, v * ab.z + a.z);
-    r.used = 3;
-    r.setBC(1.0f - v, v, 0, 0);
-    return true;
-  }
-  V3 cp = sub(p, c);
-  float d5 = dot(ab, cp), d6 = dot(ac, cp);
-  if (d6 >= 0.0f && d5 <= d6) {
-    r.closest = c; r.used = 4; r.setBC(0, 0, 1, 0);
-    return true;
-  }
-  float vb = d5 * d2 - d1 * d6;
-  if (vb <= 0.0f && d2 >= 0.0f && d6 <= 0.0f) {
-    float w = d2 / (d2 - d6);
-    r.closest = v3(w * ac.x + a.x, w * ac.y + a.y, w * ac.z + a.z);
-    r.used = 5;
-    r.setBC(1.0f - w, 0, w, 0);
-    return true;
-  }
-  float va = d3 * d6 - d5 * d4;
-  if (va <= 0.0f && (d4 - d3) >= 0.0f && (d5 - d6) >= 0.0f) {
-    float w = (d4 - d3) / ((d4 - d3) + (d5 - d6));
-    V3 t = sub(c, b);
-    r.closest = v3(w * t.x + b.x, w * t.y + b.y, w * t.z + b.z);
-    r.used = 6;
-    r.setBC(0, 1.0f - w, w, 0);
-    return true;
-  }
-  float denom = 1.0f / (va + vb + vc);
-  float v = vb * denom, w = vc * denom;
-  V3 t1 = scl(ab, v), t2 = scl(ac, w);
-  r.closest = v3(a.x + t1.x + t2.x, a.y + t1.y + t2.y, a.z + t1.z + t2.z);
-  r.used = 7;
-  r.setBC(1.0f - v - w, v, w, 0);
-  return true;
+// Closest point of triangle abc to p.  The regions are told apart by the reference's tests in its order, but only their
+// outcome is selected: lanes in different regions share the arithmetic and the one division (a vertex's is not used).
+// Branches and the four unrolled faces of a tetrahedron before this: with the hull vertices in flight (shapes.h), the pair
+// pass of a 3,001-body pile took 164 us and takes 133, 2.6 million ray casts 1.20 and 1.06 ms, 355,000 sweeps 1.9 and 1.6.
+__device__ __forceinline__ void triClosest(V3 p, V3 a, V3 b, V3 c, Sub& r) {
+  const V3 ab = sub(b, a), ac = sub(c, a), ap = sub(p, a), bp = sub(p, b), cp = sub(p, c);
+  const float d1 = dot(ab, ap), d2 = dot(ac, ap);
+  const float d3 = dot(ab, bp), d4 = dot(ac, bp);
+  const float d5 = dot(ab, cp), d6 = dot(ac, cp);
+  const float vc = d1 * d4 - d3 * d2, vb = d5 * d2 - d1 * d6, va = d3 * d6 - d5 * d4;
+  const float e4 = d4 - d3, e5 = d5 - d6;
+  const bool inA = d1 <= 0.0f && d2 <= 0.0f;
+  const bool inB = d3 >= 0.0f && d4 <= d3;
+  const bool inAB = vc <= 0.0f && d1 >= 0.0f && d3 <= 0.0f;
+  const bool inC = d6 >= 0.0f && d5 <= d6;
+  const bool inAC = vb <= 0.0f && d2 >= 0.0f && d6 <= 0.0f;
+  const bool inBC = va <= 0.0f && e4 >= 0.0f && e5 >= 0.0f;
+  // vertices used, a bit each, also the region
+  const uint32_t used = inA ? 1 : inB ? 2 : inAB ? 3 : inC ? 4 : inAC ? 5 : inBC ? 6 : 7;
+  const float num = used == 3 ? d1 : used == 5 ? d2 : used == 6 ? e4 : 1.0f;
+  const float den = used == 3 ? d1 - d3 : used == 5 ? d2 - d6 : used == 6 ? e4 + e5 : va + vb + vc;
+  const float q = num / den;
+  const bool face = used == 7, vertex = (used & (used - 1)) == 0;
+  const bool fromB = used == 2 || used == 6;
+  const V3 base = vertex ? (used == 1 ? a : used == 2 ? b : c) : fromB ? b : a;
+  const V3 bc = sub(c, b);
+  const V3 dir = used == 5 ? ac : used == 6 ? bc : ab;
+  const float v = face ? vb * q : q, w = vc * q;
+  V3 on = v3(base.x + dir.x * v, base.y + dir.y * v, base.z + dir.z * v);
+  if (face) on = v3(on.x + ac.x * w, on.y + ac.y * w, on.z + ac.z * w);
+  r.closest = vertex ? base : on;
+  r.used = used;
+  const float rest = 1.0f - v;
+  r.setBC(used == 1 ? 1.0f : used == 3 || used == 5 ? rest : face ? rest - w : 0.0f,
+          used == 2 ? 1.0f : used == 3 || face ? v : used == 6 ? rest : 0.0f,
+          used == 4 ? 1.0f : used == 5 || used == 6 ? v : face ? w : 0.0f, 0.0f);
 }
 
 __device__ __forceinline__ int outsidePlane(V3 p, V3 a, V3 b, V3 c, V3 d) {
@@ -242,49 +226,28 @@ __device__ bool tetClosest(V3 p, V3 a, V3 b, V3 c, V3 d, Sub& fr) {
     return false;
   }
   if (oABC == 0 && oACD == 0 && oADB == 0 && oBDC == 0) return false;
+  // the faces the origin is outside of (one or two as a rule) in turn, each lane its own
   float best = 3.40282347e+38f;
-  if (oABC != 0) {
-    triClosest(p, a, b, c, tr);
-    V3 t = sub(tr.closest, p);
-    float sq = dot(t, t);
+  uint32_t faces = (oABC != 0 ? 1u : 0u) | (oACD != 0 ? 2u : 0u) | (oADB != 0 ? 4u : 0u) | (oBDC != 0 ? 8u : 0u);
+  while (faces) {
+    const int f = __ffs(faces) - 1;
+    faces &= faces - 1;
+    const V3 p0 = f == 3 ? b : a, p1 = f == 0 ? b : f == 1 ? c : d, p2 = f == 1 ? d : f == 2 ? b : c;
+    triClosest(p, p0, p1, p2, tr);
+    const V3 t = sub(tr.closest, p);
+    const float sq = dot(t, t);
     if (sq < best) {
       best = sq;
       fr.closest = tr.closest;
-      fr.used = bit(tr.used, 0) | (bit(tr.used, 1) << 1) | (bit(tr.used, 2) << 2);
-      fr.setBC(tr.bc[0], tr.bc[1], tr.bc[2], 0);
-    }
-  }
-  if (oACD != 0) {
-    triClosest(p, a, c, d, tr);
-    V3 t = sub(tr.closest, p);
-    float sq = dot(t, t);
-    if (sq < best) {
-      best = sq;
-      fr.closest = tr.closest;
-      fr.used = bit(tr.used, 0) | (bit(tr.used, 1) << 2) | (bit(tr.used, 2) << 3);
-      fr.setBC(tr.bc[0], 0, tr.bc[1], tr.bc[2]);
-    }
-  }
-  if (oADB != 0) {
-    triClosest(p, a, d, b, tr);
-    V3 t = sub(tr.closest, p);
-    float sq = dot(t, t);
-    if (sq < best) {
-      best = sq;
-      fr.closest = tr.closest;
-      fr.used = bit(tr.used, 0) | (bit(tr.used, 2) << 1) | (bit(tr.used, 1) << 3);
-      fr.setBC(tr.bc[0], tr.bc[2], 0, tr.bc[1]);
-    }
-  }
-  if (oBDC != 0) {
-    triClosest(p, b, d, c, tr);
-    V3 t = sub(tr.closest, p);
-    float sq = dot(t, t);
-    if (sq < best) {
-      best = sq;
-      fr.closest = tr.closest;
-      fr.used = (bit(tr.used, 0) << 1) | (bit(tr.used, 2) << 2) | (bit(tr.used, 1) << 3);
-      fr.setBC(0, tr.bc[0], tr.bc[2], tr.bc[1]);
+      const uint32_t u0 = bit(tr.used, 0), u1 = bit(tr.used, 1), u2 = bit(tr.used, 2);
+      fr.used = f == 0 ? u0 | u1 << 1 | u2 << 2
+              : f == 1 ? u0 | u1 << 2 | u2 << 3
+              : f == 2 ? u0 | u2 << 1 | u1 << 3
+                       : u0 << 1 | u2 << 2 | u1 << 3;
+      fr.setBC(f == 3 ? 0.0f : tr.bc[0],
+               f == 0 ? tr.bc[1] : f == 1 ? 0.0f : f == 2 ? tr.bc[2] : tr.bc[0],
+               f == 0 ? tr.bc[2] : f == 1 ? tr.bc[1] : f == 2 ? 0.0f : tr.bc[2],
+               f == 0 ? 0.0f : f == 1 ? tr.bc[2] : tr.bc[1]);
     }
   }
   return true;
@@ -396,35 +359,28 @@ struct SimplexT {
           validClosest = bc.isValid();
           break;
         }
-        case 3: {
-          triClosest(v3(0, 0, 0), W(0), W(1), W(2), bc);
+        case 3:
+        case 4: {  // one tail for both: a triangle's fourth product is left out
+          const bool tet = nv == 4;
+          const V3 w0 = W(0), w1 = W(1), w2 = W(2);
+          bool apart = true;
+          if (tet) apart = tetClosest(v3(0, 0, 0), w0, w1, w2, W(3), bc);
+          else triClosest(v3(0, 0, 0), w0, w1, w2, bc);
+          if (!apart) {
+            validClosest = !bc.degenerate;
+            if (validClosest) cV = v3(0, 0, 0);
+            break;
+          }
           V3 t1 = scl(P(0), bc.bc[0]), t2 = scl(P(1), bc.bc[1]), t3 = scl(P(2), bc.bc[2]);
           cP1 = v3(t1.x + t2.x + t3.x, t1.y + t2.y + t3.y, t1.z + t2.z + t3.z);
           t1 = scl(Q(0), bc.bc[0]); t2 = scl(Q(1), bc.bc[1]); t3 = scl(Q(2), bc.bc[2]);
           cP2 = v3(t1.x + t2.x + t3.x, t1.y + t2.y + t3.y, t1.z + t2.z + t3.z);
+          if (tet) {
+            cP1 = add(cP1, scl(P(3), bc.bc[3]));
+            cP2 = add(cP2, scl(Q(3), bc.bc[3]));
+          }
           cV = sub(cP1, cP2);
           reduce(bc.used);
-          validClosest = bc.isValid();
-          break;
-        }
-        case 4: {
-          bool sep = tetClosest(v3(0, 0, 0), W(0), W(1), W(2), W(3), bc);
-          if (sep) {
-            V3 t1 = scl(P(0), bc.bc[0]), t2 = scl(P(1), bc.bc[1]), t3 = scl(P(2), bc.bc[2]), t4 = scl(P(3), bc.bc[3]);
-            cP1 = v3(t1.x + t2.x + t3.x + t4.x, t1.y + t2.y + t3.y + t4.y, t1.z + t2.z + t3.z + t4.z);
-            t1 = scl(Q(0), bc.bc[0]); t2 = scl(Q(1), bc.bc[1]); t3 = scl(Q(2), bc.bc[2]); t4 = scl(Q(3), bc.bc[3]);
-            cP2 = v3(t1.x + t2.x + t3.x + t4.x, t1.y + t2.y + t3.y + t4.y, t1.z + t2.z + t3.z + t4.z);
-            cV = sub(cP1, cP2);
-            reduce(bc.used);
-          } else {
-            if (bc.degenerate) {
-              validClosest = false;
-            } else {
-              validClosest = true;
-              cV = v3(0, 0, 0);
-            }
-            break;
-          }
           validClosest = bc.isValid();
           break;
         }
@@ -436,6 +392,24 @@ struct SimplexT {
   }
 };
 using Simplex = SimplexT<kGjkBlock>;
+
+// A wave of the pair kernel below takes every branch and as many rounds as any of its lanes, so where there are too few
+// pairs to fill the chip with full waves, waves hold fewer of them: as few as kSpreadWaves waves allow.  A 3,001-body
+// pile's pass (12,000 pairs) 133 us with full waves, 130 / 114 / 127 / 149 us at most 2048 / 4096 / 8192 / 16384 waves;
+// the simplex storage lets 3072 be resident.  From 2^18 pairs on waves are full.
+constexpr int64_t kSpreadWaves = 4096;
+inline int laneShift(int64_t n) {
+  int sh = 6;
+  while (sh > 0 && (n >> (sh - 1)) <= kSpreadWaves) sh--;
+  return sh;
+}
+inline int spreadGrid(int64_t n, int sh) { return gridFor(n, (kGjkBlock / 64) << sh); }
+// this thread's pair, or -1
+__device__ __forceinline__ int64_t spreadIndex(int sh) {
+  const int lane = threadIdx.x & 63;
+  if (lane >> sh) return -1;
+  return ((((int64_t)blockIdx.x * kGjkBlock + threadIdx.x) >> 6) << sh) + lane;
+}
 
 // ------------------------------------------------------------------ GJK pair detector
 // GjkPairDetector.getClosestPoints up to the penetration test (GjkPairDetector.java:76-260): the closest points
@@ -545,15 +519,14 @@ __device__ __forceinline__ void gjkClosest(const Shape& sa, const Tr& ta, const 
 }
 
 // epaState per pair: [needEpa, isValid, distance, pA xyz, pB xyz, nB xyz]
-// epaState per pair: [needEpa, isValid, distance, pA xyz, pB xyz, nB xyz]
 __global__ __launch_bounds__(kGjkBlock) void kGjk(const int* __restrict__ range, const int* __restrict__ list, const uint64_t* __restrict__ keys,
                                             const float* __restrict__ shapes, const float* __restrict__ verts,
                                             const float* __restrict__ props, const float* __restrict__ tr,
                                             float* cand, float* epaState, int* epaQueue,
-                                            unsigned long long* epaCount) {
+                                            unsigned long long* epaCount, int sh) {
   __shared__ float simplexLds[kSimplexRows * kGjkBlock];
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= range[1]) return;
+  const int64_t k = spreadIndex(sh);
+  if (k < 0 || k >= range[1]) return;
   int i = list[range[0] + k];
   int a = (int)(keys[i] >> 32) - 1, b = (int)(keys[i] & 0xffffffffu) - 1;
   Shape sa = bodyShape(shapes, props, a), sb = bodyShape(shapes, props, b);
@@ -2223,9 +2196,10 @@ void npDispatchAll(Ctx& c) {
   hipLaunchKernelGGL(kConvexPlane, dim3(gridFor(n)), dim3(256), 0, s, (const int*)range + 2 * JBGPU_PAIR_CONVEX_PLANE,
                      list, keys, c.shapes.p, c.verts.p, c.props.p, c.tr.p, c.candC.p);
   tBegin(c, T_GJK);
-  hipLaunchKernelGGL(kGjk, dim3(gridFor(n, kGjkBlock)), dim3(kGjkBlock), 0, s,
+  const int sh = laneShift(n);
+  hipLaunchKernelGGL(kGjk, dim3(spreadGrid(n, sh)), dim3(kGjkBlock), 0, s,
                      (const int*)range + 2 * JBGPU_PAIR_CONVEX_CONVEX, list, keys, c.shapes.p, c.verts.p, c.props.p,
-                     c.tr.p, c.candC.p, c.epaState.p, c.epaQueue.p, c.npStat.p);
+                     c.tr.p, c.candC.p, c.epaState.p, c.epaQueue.p, c.npStat.p, sh);
   tEnd(c, T_GJK);
   tBegin(c, T_EPA);
   c.epaRetry.ensure(n);
@@ -2288,9 +2262,10 @@ void npDispatchGraph(Ctx& c) {
                      list, keys, c.shapes.p, c.props.p, c.tr.p, c.candC.p);
   hipLaunchKernelGGL(kConvexPlane, dim3(gridFor(n)), dim3(256), 0, s, (const int*)range + 2 * JBGPU_PAIR_CONVEX_PLANE,
                      list, keys, c.shapes.p, c.verts.p, c.props.p, c.tr.p, c.candC.p);
-  hipLaunchKernelGGL(kGjk, dim3(gridFor(n, kGjkBlock)), dim3(kGjkBlock), 0, s,
+  const int sh = laneShift(n);
+  hipLaunchKernelGGL(kGjk, dim3(spreadGrid(n, sh)), dim3(kGjkBlock), 0, s,
                      (const int*)range + 2 * JBGPU_PAIR_CONVEX_CONVEX, list, keys, c.shapes.p, c.verts.p, c.props.p,
-                     c.tr.p, c.candC.p, c.epaState.p, c.epaQueue.p, c.npStat.p);
+                     c.tr.p, c.candC.p, c.epaState.p, c.epaQueue.p, c.npStat.p, sh);
   hipLaunchKernelGGL(kEpaSmall, dim3(kEpaSmallGrid), dim3(64), 0, s, (const unsigned long long*)c.npStat.p,
                      (const int*)c.epaQueue.p, keys, c.shapes.p, c.verts.p, c.props.p, c.tr.p, c.epaState.p, c.candC.p,
                      c.npStat.p + 1, c.epaRetry.p, c.npStat.p + 3, c.epaSmallFaces);

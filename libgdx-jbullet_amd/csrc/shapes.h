@@ -61,12 +61,22 @@ JBD V3 hullSupport(const float* verts, int first, int n, V3 vec) {
   else
     vec = scl(vec, 1.0f / jsqrt(l2));
   const float* p = verts + 3 * first;
-  for (int i = 0; i < n; i++) {
-    V3 vtx = v3(p[3 * i] * 1.0f, p[3 * i + 1] * 1.0f, p[3 * i + 2] * 1.0f);
-    float d = dot(vec, vtx);
-    if (d > maxDot) {
-      maxDot = d;
-      sup = vtx;
+  // eight vertices in flight at a time; past the end the last one again, which is never greater than itself
+  constexpr int U = 8;
+  for (int i = 0; i < n; i += U) {
+    V3 w[U];
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      const float* q = p + 3 * (i + k < n ? i + k : n - 1);
+      w[k] = v3(q[0] * 1.0f, q[1] * 1.0f, q[2] * 1.0f);
+    }
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      const float d = dot(vec, w[k]);
+      if (d > maxDot) {
+        maxDot = d;
+        sup = w[k];
+      }
     }
   }
   return sup;
