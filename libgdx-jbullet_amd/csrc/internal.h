@@ -281,7 +281,7 @@ struct Ctx {
   DBuf<int> typeKey, typeKeyAlt, perm, permAlt;
   DBuf<unsigned long long> npStat;           // EPA queue length, failures, workspace overflows
   DBuf<int> binRange;                        // per pair type: first sorted position and count
-  unsigned long long npStatHost[5] = {0, 0, 0, 0, 0};  // their copy, valid after the step's final synchronisation
+  HBuf<unsigned long long> npStatHost;  // their copy, valid after the step's final synchronisation
   bool npStatPending = false;
   bool epaOverflow = false;  // the last narrowphase pass overflowed an EPA workspace
   std::vector<int> shapeTypeHost;  // host copies: type per shape and per body (canonical manifold headers)
@@ -323,9 +323,10 @@ struct Ctx {
   HBuf<double> solveRh;               // per-iteration (change, norm) sums
   HBuf<unsigned long long> solveRows; // rows in total, rows of the per-colour or block sweeps
   struct {
-    bool pending = false, tolMode = false, blockSweeps = false, sampleK = false, flow = false;
+    bool pending = false, toCopy = false, tolMode = false, blockSweeps = false, sampleK = false, flow = false;
     int iters = 0, sampledIters = 0;  // sampledIters: iterations whose sweep launches were event-timed
     size_t kUsed = 0;
+    const int* flowErr = nullptr;
   } solveStat;
   DBuf<float> candC;  // contact candidates npairs*8
   DBuf<int> epaQueue;
@@ -348,7 +349,6 @@ struct Ctx {
   HBuf<int> flowErrHost;
   bool oddBodies = false;  // a body flagged static has a mass
   // slot order of a small step: its counts and colour starts, and the last step's manifolds
-  DBuf<int> smallInfo;
   HBuf<int> smallInfoHost;
   int64_t smallTooMany = 0;
   DBuf<int2> activeBodies;   // per active manifold: body A, body B
@@ -483,6 +483,21 @@ struct FillList {  // several fills in one launch
   }
 };
 void graphFillList(hipStream_t s, const FillList& f);
+struct CopyList {  // several small copies in one launch, device memory to device-visible memory
+  static constexpr int kMax = 8;
+  uint32_t* dst[kMax];
+  const uint32_t* src[kMax];
+  uint32_t n[kMax];
+  int count = 0;
+  void add(void* to, const void* from, size_t bytes) {
+    if (count >= kMax) throw std::logic_error("copy list full");
+    dst[count] = (uint32_t*)to;
+    src[count] = (const uint32_t*)from;
+    n[count] = (uint32_t)(bytes / 4);
+    count++;
+  }
+};
+void copyList(hipStream_t s, const CopyList& f);
 void bpGraphReserve(Ctx& c);
 const uint64_t* bpStepGraph(Ctx& c);  // AABB update, tree, traversal, key sort; returns the sorted keys
 void bpRemapGraph(Ctx& c, const uint64_t* sorted);
@@ -497,6 +512,7 @@ void bpPairDeltas(Ctx& c, uint64_t* added, int64_t capAdded, int64_t* nAdded, ui
 void npDispatchAll(Ctx& c);                              // A8-A16
 int64_t npCountContacts(Ctx& c);                         // contact points of the current manifolds
 void npCollectStats(Ctx& c);                             // EPA statistics of the last narrowphase
+void statsCopy(Ctx& c);  // whatever the step left to collect, into pinned memory; before its final synchronisation
 void solverCollectStats(Ctx& c);                         // residual, rows and sweep timings of the last solve
 // solver
 // A18-A20; explicit: the manifolds to solve (pair indices, the islands a caller recorded) instead of the
@@ -554,6 +570,7 @@ void primScan(Ctx& c, const int* in, int* out, int n);
 // the same with the element count in device memory (*count, at most cap): launches shaped by cap only, as a
 // captured graph needs; the sorted data ends in k.cur / v.cur (which buffer that is depends on cap and the bits)
 void primReserve(Ctx& c, int cap);  // scratch for counts up to cap, allocated outside a capture
+const int* primErrWord(Ctx& c);  // the sorts' error word on the device (null: no sort yet), its host copy cleared
 void primErrCopy(Ctx& c);   // the sorts' error word into pinned memory (asynchronous)
 void primErrCheck(Ctx& c);  // after the stream's wait: throws if a sort's look-back gave up
 template <class K>

@@ -487,11 +487,14 @@ void primScan(Ctx& c, const int* in, int* out, int n) {
 // ---- device-count forms (graph-captured steps) -----------------------------------------------------------------
 void primReserve(Ctx& c, int cap) { (void)primScratch(c, std::max(cap, 1)); }
 
-void primErrCopy(Ctx& c) {
+const int* primErrWord(Ctx& c) {
   c.primErrHost.ensure(1);
   c.primErrHost.p[0] = 0;
-  if (c.primTmp.p)
-    JB_CHECK(hipMemcpyAsync(c.primErrHost.p, c.primTmp.p + kHdrErr, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+  return c.primTmp.p ? (const int*)(c.primTmp.p + kHdrErr) : nullptr;
+}
+void primErrCopy(Ctx& c) {
+  if (const int* err = primErrWord(c))
+    JB_CHECK(hipMemcpyAsync(c.primErrHost.p, err, sizeof(int), hipMemcpyDeviceToHost, c.stream));
 }
 void primErrCheck(Ctx& c) {
   if (c.primErrHost.p && c.primErrHost.p[0])
@@ -545,6 +548,18 @@ void graphFillList(hipStream_t s, const FillList& f) {
   for (int e = 0; e < f.count; e++) most = std::max(most, f.n[e]);
   const int grid = (int)std::min<uint32_t>((most + 255) / 256, 256);
   hipLaunchKernelGGL(kFillList, dim3(std::max(grid, 1)), dim3(256), 0, s, f);
+}
+// a copy command each takes 2 to 5 us on the stream and as long to queue; a step's end has up to six of them
+__global__ void kCopyList(CopyList f) {
+  for (int e = 0; e < f.count; e++)
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < f.n[e]; i += gridDim.x * blockDim.x)
+      f.dst[e][i] = f.src[e][i];
+}
+void copyList(hipStream_t s, const CopyList& f) {
+  if (f.count == 0) return;
+  uint32_t most = 0;
+  for (int e = 0; e < f.count; e++) most = std::max(most, f.n[e]);
+  hipLaunchKernelGGL(kCopyList, dim3(std::min<uint32_t>((most + 255) / 256, 64)), dim3(256), 0, s, f);
 }
 void graphFill(hipStream_t s, void* p, size_t words, uint32_t v) {
   if (words == 0) return;

@@ -1204,8 +1204,8 @@ typedef unsigned long long flow_t;
 constexpr int kFlowShards = 16;
 // control words (ints, 128 bytes apart): starting order, one ticket counter per sequence, error (sticky)
 constexpr int kFlowCtlTicket = 32, kFlowCtlStride = 32;
-constexpr int kFlowCtlErr = kFlowCtlTicket + kFlowCtlStride * kFlowShards;
-constexpr int kFlowCtlWords = kFlowCtlErr + kFlowCtlStride;
+constexpr int kFlowCtlWords = kFlowCtlTicket + kFlowCtlStride * kFlowShards;  // of one launch
+constexpr int kFlowCtls = 64;  // launches whose words are cleared together
 constexpr int kFlowMaxColours = 64;
 constexpr int kFlowSlots = 16;           // slots per group (one wave, four lanes per slot)
 constexpr int kFlowSpinLimit = 1 << 22;  // polls of one group (about a microsecond each)
@@ -1240,9 +1240,9 @@ __global__ void kFlowInit(int na, int nb, const int4* __restrict__ hdr, const in
                           const int* __restrict__ color, const unsigned long long* __restrict__ bodyMask,
                           const float* __restrict__ props, const float* __restrict__ svel,
                           const float* __restrict__ nrow, const float* __restrict__ frow, int4* dep, flow_t* napp,
-                          flow_t* fapp, flow_t* body, int* ctl) {
+                          flow_t* fapp, flow_t* body, int* ctl, int ctlWords) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < kFlowCtlWords) ctl[t] = 0;
+  if (t < ctlWords) ctl[t] = 0;
   if (t < nb) {
     const float4* s = (const float4*)(svel + 8 * (size_t)t);
     const float4 a = s[0], b = s[1];
@@ -1277,7 +1277,8 @@ struct FlowSweep {
   flow_t* fapp;
   flow_t* body;
   float* svel;
-  int* ctl;
+  int* ctl;  // the launch's tickets
+  int* err;
 };
 // the group a wave works on: the quad's slot (none: valid false) in sweep `sweep` of the launch
 struct FlowGroup {
@@ -1487,7 +1488,7 @@ __device__ __forceinline__ bool flowRun(const FlowSweep& W, const SolverParams& 
     pending = pending && !go;
     if (!__any(pending)) return true;
     if (spin >= kFlowSpinLimit) return false;
-    if ((spin & 1023) == 1023 && __hip_atomic_load(W.ctl + kFlowCtlErr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    if ((spin & 1023) == 1023 && __hip_atomic_load(W.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       return false;
     const bool near = ((__ballot(away <= 1) >> (lane & ~3)) & 15) == 15;
     if (!__any(pending && near)) __builtin_amdgcn_s_sleep(8);
@@ -1546,7 +1547,7 @@ __global__ __launch_bounds__(64) void kFlowSweep(int na, int ncol, const int* __
     const bool ok = w & 1 ? flowRun<true>(W, SP, G, it, it == trackIt, last, dd, nn)
                                 : flowRun<false>(W, SP, G, it, it == trackIt, last, dd, nn);
     if (!ok) {
-      if (lane == 0) atomicOr(W.ctl + kFlowCtlErr, 1);
+      if (lane == 0) atomicOr(W.err, 1);
       break;
     }
     G = N;
@@ -2708,6 +2709,7 @@ void solveWorldBlocks(Ctx& c, float dt, int na, const int* dna = nullptr) {
   if (iters > 0)
     JB_CHECK(hipMemcpyAsync(c.solveRh.p, c.resid.p, 2 * (size_t)iters * sizeof(double), hipMemcpyDeviceToHost, s));
   JB_CHECK(hipMemcpyAsync(c.solveRows.p, c.rowCount.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+  c.solveStat.toCopy = false;
   JB_CHECK(hipMemcpyAsync(c.wbInfoHost.p, c.wbInfo.p, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
   c.solveStat.pending = true;
   c.solveStat.tolMode = false;
@@ -2779,14 +2781,12 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
     c.bodyMask.ensure(c.nb);
     c.colorStart.ensure(64);
     c.rowCount.ensure(2);
-    c.smallInfo.ensure(kSmallInfo);
     c.smallInfoHost.ensure(kSmallInfo);
     tBegin(c, T_COLOR);
     hipLaunchKernelGGL(kSmallOrder, dim3(1), dim3(kSmallThreads), 0, s, (int)np, given, flags, (const float*)man,
                        (const float*)c.props.p, c.nb, c.mActive.p, c.color.p, c.colorOrder.p, c.bodyMask.p,
-                       c.colorStart.p, c.slotCount.p, c.slotStart.p, c.rowCount.p, c.smallInfo.p);
+                       c.colorStart.p, c.slotCount.p, c.slotStart.p, c.rowCount.p, c.smallInfoHost.p);
     tEnd(c, T_COLOR);
-    JB_CHECK(hipMemcpyAsync(c.smallInfoHost.p, c.smallInfo.p, kSmallInfo * sizeof(int), hipMemcpyDeviceToHost, s));
     JB_CHECK(hipStreamSynchronize(s));
     ordered = c.smallInfoHost.p[0] == 0;
     return c.smallInfoHost.p[1];
@@ -3105,11 +3105,27 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
                      blockSweeps ? (int)c.interiorEnd : (int)c.colorOff[headColors], (const int*)c.slotCount.p,
                      (const int*)c.slotStart.p, c.rowCount.p);
   if (learnedHere) mlpWarmStart(c, na);  // overwrites the applied words of the valid rows
+  // The residual is accumulated only where it is used: every iteration in tolerance mode, else the last one.
+  const bool tolMode = c.tolerance > 0.0f;
+  int iters = tolMode ? c.maxIterations : c.numIterations;
+  const size_t histWords = 2 * (size_t)iters + 4, stripeWords = 2 * (size_t)kResidStripes * iters;
+  c.resid.ensure(histWords + stripeWords);
+  c.done.ensure(4);
+  float* resOut = (float*)(c.counter.p + 6);
+  FillList fills;  // what the solve accumulates into, cleared with the warm start's table where there is one
+  fills.add(c.resid.p, 2 * (histWords + stripeWords), 0u);
+  fills.add(c.done.p, 4, 0u);
+  fills.add(resOut, 2, 0u);
   const bool apply = c.warmstart || c.useLearned || c.useMlp;
   int setupLaunches = 1;
   if (apply && !blockSweeps && c.ncolors <= kWarmGatherBatches) {  // warm start gathered per body
-    c.warmSlotOf.ensure((size_t)c.ncolors * c.nb);
-    JB_CHECK(hipMemsetAsync(c.warmSlotOf.p, 0xff, (size_t)c.ncolors * c.nb * sizeof(int), s));
+    constexpr size_t kFillListWords = 1 << 18;  // a longer table is cleared faster by a fill of its own
+    const size_t words = (size_t)c.ncolors * c.nb;
+    c.warmSlotOf.ensure(words);
+    if (words <= kFillListWords) fills.add(c.warmSlotOf.p, words, 0xffffffffu);
+    else JB_CHECK(hipMemsetAsync(c.warmSlotOf.p, 0xff, words * sizeof(int), s));
+    graphFillList(s, fills);
+    fills.count = 0;
     hipLaunchKernelGGL(kWarmSlotTable, dim3(gridFor(na)), dim3(256), 0, s, na, c.ncolors, (const int*)c.colorStart.p,
                        (const int4*)c.hdr.p, (const float*)c.svel.p, c.nb, c.warmSlotOf.p);
     hipLaunchKernelGGL(kWarmGather, dim3(gridFor(c.nb)), dim3(256), 0, s, c.nb, c.ncolors,
@@ -3129,16 +3145,7 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   }
   tEnd(c, T_SOLVE_SETUP, setupLaunches);
   // iterations
-  // The residual is accumulated only where it is used: every iteration in tolerance mode, else the last one.
-  const bool tolMode = c.tolerance > 0.0f;
-  int iters = tolMode ? c.maxIterations : c.numIterations;
-  const size_t histWords = 2 * (size_t)iters + 4, stripeWords = 2 * (size_t)kResidStripes * iters;
-  c.resid.ensure(histWords + stripeWords);
-  c.done.ensure(4);
-  JB_CHECK(hipMemsetAsync(c.resid.p, 0, (histWords + stripeWords) * sizeof(double), s));
-  JB_CHECK(hipMemsetAsync(c.done.p, 0, 4 * sizeof(int), s));
-  float* resOut = (float*)(c.counter.p + 6);
-  JB_CHECK(hipMemsetAsync(resOut, 0, 2 * sizeof(float), s));
+  graphFillList(s, fills);  // unless done above
   int* done = tolMode ? c.done.p : nullptr;
   // kernel-level timing of this step's sweeps (sampled): on a sampled step, the launches of every
   // kernelStride-th iteration get their own events (every iteration sweeps the same colours and rows; the events
@@ -3190,6 +3197,11 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   int launchedIters = iters;
   if (tolMode) c.doneHost.ensure(1);
   int64_t flowLaunches = 0;
+  const bool oneLaunch = flow && !tolMode && !jp.on && !sampleK && iters > 0;
+  const int flowCtls = oneLaunch ? 1 : std::min(2 * std::max(iters, 1), kFlowCtls);
+  const int flowCtlWords = flowCtls * kFlowCtlWords + 1;
+  if (flow) c.flowCtl.ensure(flowCtlWords);
+  int* flowErr = flow ? c.flowCtl.p + flowCtlWords - 1 : nullptr;
   // one launch of `sweeps` sweeps from sweep0 on; timed: with its own events
   auto flowSweep = [&](int sweep0, int sweeps, double* res, bool timed) {
     // Waves beyond what the dependences keep busy only poll (their reads go past the L2).  Solve time by grid:
@@ -3198,9 +3210,11 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
     const int groups = na / kFlowSlots + c.ncolors;  // at least the groups of a sweep
     const int grid = std::min(1536, std::max(128, groups / 2));
     static_assert(kFlowShards <= 128, "every ticket sequence needs a workgroup");
-    if (sweep0 > 0) JB_CHECK(hipMemsetAsync(c.flowCtl.p, 0, kFlowCtlErr * sizeof(int), s));  // not the error word
+    const int ctl = (int)(flowLaunches % flowCtls);
+    if (flowLaunches > 0 && ctl == 0)  // not the error word behind them
+      JB_CHECK(hipMemsetAsync(c.flowCtl.p, 0, (size_t)flowCtls * kFlowCtlWords * sizeof(int), s));
     const FlowSweep W{c.hdr.p, c.flowDep.p, c.nrow.p, c.frow.p, c.flowNapp.p, c.flowFapp.p, c.flowBody.p, c.svel.p,
-                      c.flowCtl.p};
+                      c.flowCtl.p + (size_t)ctl * kFlowCtlWords, flowErr};
     const int trackIt = res ? (sweep0 + sweeps - 1) >> 1 : -1;
     if (timed) {
       hipEvent_t* ev = kPair(sweep0 & 1);
@@ -3217,14 +3231,12 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
     c.flowNapp.ensure(4 * (size_t)na);
     c.flowFapp.ensure(8 * (size_t)na);
     c.flowBody.ensure(4 * (size_t)c.nb);
-    c.flowCtl.ensure(kFlowCtlWords);
-    hipLaunchKernelGGL(kFlowInit, dim3(gridFor(std::max<int64_t>({4 * (int64_t)na, c.nb, kFlowCtlWords}))), dim3(256), 0,
+    hipLaunchKernelGGL(kFlowInit, dim3(gridFor(std::max<int64_t>({4 * (int64_t)na, c.nb, flowCtlWords}))), dim3(256), 0,
                        s, na, c.nb, (const int4*)c.hdr.p, (const int*)c.colorOrder.p, (const int*)c.color.p,
                        (const unsigned long long*)c.bodyMask.p, (const float*)c.props.p, (const float*)c.svel.p,
                        (const float*)c.nrow.p, (const float*)c.frow.p, c.flowDep.p, c.flowNapp.p, c.flowFapp.p,
-                       c.flowBody.p, c.flowCtl.p);
+                       c.flowBody.p, c.flowCtl.p, flowCtlWords);
   }
-  const bool oneLaunch = flow && !tolMode && !jp.on && !sampleK && iters > 0;
   if (oneLaunch) {
     double* res = c.resid.p + histWords + 2 * (size_t)kResidStripes * (iters - 1);
     flowSweep(0, 2 * iters, res, false);
@@ -3297,18 +3309,14 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
            jointLaunches);
   hipLaunchKernelGGL(kWriteback, dim3(gridFor(na)), dim3(256), 0, s, na, (const int*)nullptr, c.hdr.p, c.nrow.p, c.frow.p, man);
   hipLaunchKernelGGL(kCopyVel, dim3(gridFor(c.nb)), dim3(256), 0, s, c.nb, c.svel.p, c.vel.p, c.props.p);
-  // statistics: copied into pinned memory now, read by solverCollectStats after the step's final wait
+  // statistics: copied by statsCopy, read by solverCollectStats after the step's final wait
   c.solveRo.ensure(2);
   c.solveRh.ensure(2 * (size_t)std::max(iters, 1));
   c.solveRows.ensure(2);
-  JB_CHECK(hipMemcpyAsync(c.solveRo.p, resOut, 2 * sizeof(float), hipMemcpyDeviceToHost, s));
-  if (iters > 0)
-    JB_CHECK(hipMemcpyAsync(c.solveRh.p, c.resid.p, 2 * (size_t)iters * sizeof(double), hipMemcpyDeviceToHost, s));
-  JB_CHECK(hipMemcpyAsync(c.solveRows.p, c.rowCount.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   c.flowErrHost.ensure(1);
   c.flowErrHost.p[0] = 0;
-  if (flow)
-    JB_CHECK(hipMemcpyAsync(c.flowErrHost.p, c.flowCtl.p + kFlowCtlErr, sizeof(int), hipMemcpyDeviceToHost, s));
+  c.solveStat.flowErr = flowErr;
+  c.solveStat.toCopy = true;
   c.solveStat.pending = true;
   c.solveStat.flow = flow;
   c.solveStat.tolMode = tolMode;
@@ -3317,6 +3325,20 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   c.solveStat.sampledIters = sampledIters;
   c.solveStat.iters = iters;
   c.solveStat.kUsed = kUsed;
+}
+
+void statsCopy(Ctx& c) {
+  CopyList f;
+  if (c.npStatPending) f.add(c.npStatHost.p, c.npStat.p, 5 * sizeof(unsigned long long));
+  if (c.solveStat.pending && c.solveStat.toCopy) {
+    f.add(c.solveRo.p, c.counter.p + 6, 2 * sizeof(float));
+    f.add(c.solveRh.p, c.resid.p, 2 * (size_t)c.solveStat.iters * sizeof(double));
+    f.add(c.solveRows.p, c.rowCount.p, 2 * sizeof(unsigned long long));
+    if (c.solveStat.flowErr) f.add(c.flowErrHost.p, c.solveStat.flowErr, sizeof(int));
+    c.solveStat.toCopy = false;
+  }
+  if (const int* err = primErrWord(c)) f.add(c.primErrHost.p, err, sizeof(int));
+  copyList(c.stream, f);
 }
 
 void solverCollectStats(Ctx& c) {

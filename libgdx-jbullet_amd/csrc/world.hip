@@ -399,7 +399,7 @@ void stepPhases(Ctx& c, float dt, int last) {
                        c.props.p, c.act.p, c.deact.p, c.vel.p, (const int*)nullptr);
   }
   tEnd(c, T_STEP);
-  primErrCopy(c);
+  statsCopy(c);
   JB_CHECK(hipStreamSynchronize(s));
   primErrCheck(c);
   npCollectStats(c);
@@ -501,6 +501,7 @@ void stepAfterAabbs(Ctx& c, float dt) {
   ccdClamp(c, dt);
   hipLaunchKernelGGL(kActivation, dim3(gridFor(c.nb)), dim3(256), 0, s, c.nb, dt, c.deactivationDisabled, c.props.p,
                      c.act.p, c.deact.p, c.vel.p, (const int*)nullptr);
+  statsCopy(c);
   JB_CHECK(hipStreamSynchronize(s));
   npCollectStats(c);
   solverCollectStats(c);
@@ -1482,6 +1483,7 @@ int jbgpu_np_dispatch(jbgpu_ctx* ctx, int64_t n, const uint64_t* keys, const flo
     canonicalHeaders(c, n, keys, man.data());
     uploadPairs(c, n, keys, man.data());
     npDispatchAll(c);
+    statsCopy(c);
     JB_CHECK(hipStreamSynchronize(c.stream));
     npCollectStats(c);
     if (n)
@@ -1527,6 +1529,7 @@ int jbgpu_solver_all_solved(jbgpu_ctx* ctx, float dt) {
       seen[k] = 1;
     }
     solverSolve(c, dt, &c.islandManifolds);
+    statsCopy(c);
     JB_CHECK(hipStreamSynchronize(c.stream));
     solverCollectStats(c);
   });

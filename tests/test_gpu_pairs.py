@@ -92,3 +92,25 @@ def test_proxies_destroyed_between_set_aabb_and_the_query(n):
     assert len(got) and not (np.isin(lo, dead) | np.isin(hi, dead)).any()
     assert np.array_equal(got, orc.step())
     ctx.close()
+
+
+@pytest.mark.parametrize("couples", [(0, 1, 2, 3), (4095, 4096, 4097, 4096), (5000, 10, 1025, 1024)])
+def test_pair_counts_around_the_small_sort(couples):
+    """Exactly so many pairs in successive queries (the first of a size is met with the expectation of the last), uids
+    shuffled; the sorted keys are known."""
+    rng = np.random.default_rng(5)
+    most = max(couples)
+    c = np.repeat(np.stack([np.arange(most) * 4.0, np.zeros(most), np.zeros(most)], 1), 2, 0).astype(np.float32)
+    perm = rng.permutation(2 * most)
+    place = np.argsort(perm)  # body of couple k: uids place[2k] + 1, place[2k + 1] + 1
+    ctx = jbgpu.Context(bp_mode=jbgpu.BP_DBVT, world_min=WMIN, world_max=WMAX)
+    half = np.float32(0.5)
+    ctx.bp_create_proxies(np.concatenate([c - half, c + half], 1)[perm])
+    for k in couples:
+        d = c.copy()
+        d[2 * k + 1::2, 1] = 50.0  # the other couples come apart
+        ctx.bp_set_aabbs(np.concatenate([d - half, d + half], 1).astype(np.float32)[perm])
+        ctx.bp_calculate_overlapping_pairs()
+        u = np.sort(place[:2 * k].reshape(-1, 2) + 1, 1).astype(np.uint64)
+        assert np.array_equal(ctx.bp_pairs(), np.sort(u[:, 0] << np.uint64(32) | u[:, 1]))
+    ctx.close()
