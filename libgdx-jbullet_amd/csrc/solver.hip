@@ -1292,62 +1292,74 @@ struct FlowGroup {
 // four products meet by DPP; the scalars of row L sit in lane L.  A row costs its dot product, two DPP steps and one
 // update per lane, about 30 instructions, where one lane doing a whole row (and handing both bodies on to the next
 // point's lane) took about 70: on the critical path of a body with many slots that is time per update.
-__device__ __forceinline__ float quadPairSum(float x) {  // x of this lane and of its neighbour (lanes 0/1, 2/3)
-  return x + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xf, 0xf, false));
+//
+// Rows run without branches of their own: a lane whose body does not move, or whose quad has no such row, keeps its
+// values by selection.  What does not depend on the velocities (the row's scalars, from their lane to the quad) is spread
+// before the wait.  With a branch per clamp, body and point the solves took 212 us (1.3k slots, 10 iterations), 1.09 ms
+// (7.1k slots) and 2.43 ms (243k); 185 us, 1.03 and 2.34 ms without.
+template <int Ctrl>
+__device__ __forceinline__ float quadPerm(float x) {  // quads are active as a whole; this form merges into its user
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), Ctrl, 0xf, 0xf, true));
 }
 __device__ __forceinline__ float flowRelVel(V3 D, V3 v) {  // (nrm.A.lv + r1.A.av) - (nrm.B.lv + r2.B.av)
-  const float s = quadPairSum(dot(D, v));
-  return quadBcast<0>(s) - quadBcast<2>(s);
+  float s = dot(D, v);
+  s = s + quadPerm<0xB1>(s);  // lanes 0 and 1, 2 and 3
+  return quadPerm<0x00>(s) - quadPerm<0xAA>(s);
 }
-__device__ __forceinline__ void flowApply(V3& v, V3 U, float imp, int q, bool moves) {
-  const float m = q < 2 ? imp : -imp;
-  if (moves) {
-    v.x += m * U.x;
-    v.y += m * U.y;
-    v.z += m * U.z;
-  }
+// U has the sign of the lane's body
+__device__ __forceinline__ void flowApply(V3& v, V3 U, float imp, bool moves) {
+  const V3 n = v3(v.x + imp * U.x, v.y + imp * U.y, v.z + imp * U.z);
+  v = v3(moves ? n.x : v.x, moves ? n.y : v.y, moves ? n.z : v.z);
 }
 // normal row of point L: resolveSingleCollisionCombinedCacheFriendly (:234-284)
 template <int L>
-__device__ __forceinline__ void flowNormalRound(int q, int nr, bool moves, const V3* D, const V3* U, float pimp,
-                                                float rest, float jac, float old, V3& v, float& out) {
-  if (!__any(nr > L)) return;
-  if (nr > L) {
-    const float velocityError = quadBcast<L>(rest) - flowRelVel(D[L], v);
-    const float vimp = velocityError * quadBcast<L>(jac);
-    float ni = quadBcast<L>(pimp) + vimp;
-    const float was = quadBcast<L>(old);
-    const float sum = was + ni;
-    const float nw = 0.0f > sum ? 0.0f : sum;
-    ni = nw - was;
-    flowApply(v, U[L], ni, q, moves);
-    if (q == L) out = nw;
-  }
+__device__ __forceinline__ void flowNormalRound(int most, int q, int nr, bool moves, const V3* D, const V3* U,
+                                                const float* pimp, const float* rest, const float* jac, float old, V3& v,
+                                                float& out) {
+  if (L >= most) return;
+  const bool row = nr > L;
+  const float velocityError = rest[L] - flowRelVel(D[L], v);
+  const float vimp = velocityError * jac[L];
+  float ni = pimp[L] + vimp;
+  const float was = quadBcast<L>(old);
+  const float sum = was + ni;
+  const float nw = 0.0f > sum ? 0.0f : sum;
+  ni = nw - was;
+  flowApply(v, U[L], ni, moves && row);
+  out = q == L && row ? nw : out;
 }
 // one friction row of point L: resolveSingleFrictionCacheFriendly (:286-346)
-template <int L>
-__device__ __forceinline__ void flowFrictionRow(int q, bool moves, V3 D, V3 U, float total, float fric, float jac,
-                                                float old, V3& v, float& out) {
-  const float limit = quadBcast<L>(total) * quadBcast<L>(fric);
-  const float j1 = -flowRelVel(D, v) * quadBcast<L>(jac);
-  const float was = quadBcast<L>(old);
-  float ap = was + j1;
-  if (limit < ap) {
-    ap = limit;
-  } else if (ap < -limit) {
-    ap = -limit;
-  }
-  flowApply(v, U, ap - was, q, moves);
-  if (q == L) out = ap;
+__device__ __forceinline__ void flowFrictionRow(bool mine, bool moves, V3 D, V3 U, float limit, float jac, float was, V3& v,
+                                                float& out) {
+  const float j1 = -flowRelVel(D, v) * jac;
+  const float to = was + j1;
+  const float low = to < -limit ? -limit : to;
+  const float ap = limit < to ? limit : low;
+  flowApply(v, U, ap - was, moves);
+  out = mine ? ap : out;
 }
 template <int L>
-__device__ __forceinline__ void flowFrictionRound(int q, int nr, bool moves, const V3* D, const V3* U, float total,
-                                                  float fric0, float jac0, float old0, float fric1, float jac1,
-                                                  float old1, V3& v, float& out0, float& out1) {
-  if (!__any(nr > L)) return;
-  if (nr > L && quadBcast<L>(total) > 0.0f) {
-    flowFrictionRow<L>(q, moves, D[2 * L], U[2 * L], total, fric0, jac0, old0, v, out0);
-    flowFrictionRow<L>(q, moves, D[2 * L + 1], U[2 * L + 1], total, fric1, jac1, old1, v, out1);
+__device__ __forceinline__ void flowFrictionRound(int most, int q, int nr, bool moves, const V3* D, const V3* U,
+                                                  float total, const float* fric, const float* jac, float old0, float old1,
+                                                  V3& v, float& out0, float& out1) {
+  if (L >= most) return;
+  const float sum = quadBcast<L>(total);
+  const bool row = nr > L && sum > 0.0f, move = moves && row, mine = q == L && row;
+  flowFrictionRow(mine, move, D[2 * L], U[2 * L], sum * fric[2 * L], jac[2 * L], quadBcast<L>(old0), v, out0);
+  flowFrictionRow(mine, move, D[2 * L + 1], U[2 * L + 1], sum * fric[2 * L + 1], jac[2 * L + 1], quadBcast<L>(old1), v,
+                  out1);
+}
+
+template <bool Fr>
+__device__ __forceinline__ void spreadScalars(float s15, float s16, float s17, float s18, float* jac, float* coef) {
+  if (Fr) {
+    jac[0] = quadBcast<0>(s15); jac[2] = quadBcast<1>(s15); jac[4] = quadBcast<2>(s15); jac[6] = quadBcast<3>(s15);
+    jac[1] = quadBcast<0>(s17); jac[3] = quadBcast<1>(s17); jac[5] = quadBcast<2>(s17); jac[7] = quadBcast<3>(s17);
+    coef[0] = quadBcast<0>(s16); coef[2] = quadBcast<1>(s16); coef[4] = quadBcast<2>(s16); coef[6] = quadBcast<3>(s16);
+    coef[1] = quadBcast<0>(s18); coef[3] = quadBcast<1>(s18); coef[5] = quadBcast<2>(s18); coef[7] = quadBcast<3>(s18);
+  } else {
+    jac[0] = quadBcast<0>(s15); jac[1] = quadBcast<1>(s15); jac[2] = quadBcast<2>(s15); jac[3] = quadBcast<3>(s15);
+    coef[0] = quadBcast<0>(s17); coef[1] = quadBcast<1>(s17); coef[2] = quadBcast<2>(s17); coef[3] = quadBcast<3>(s17);
   }
 }
 
@@ -1372,7 +1384,8 @@ __device__ __forceinline__ bool flowRun(const FlowSweep& W, const SolverParams& 
   float s15 = 0.0f, s16 = 0.0f, s17 = 0.0f, s18 = 0.0f;  // normal: jacInv, pen, rest; friction: jacInv and fric of both
   {
     const int od = q == 1 ? 3 : q == 3 ? 6 : 0, ou = q == 1 ? 9 : q == 3 ? 12 : 0;
-    const float scale = q & 1 ? 1.0f : invMass;  // linear: the normal times the inverse mass
+    // linear: the normal times the inverse mass; body B's impulse is the negative one
+    const float scale = (q & 1 ? 1.0f : invMass) * (q < 2 ? 1.0f : -1.0f);
     const float* rows = (Fr ? W.frow + (size_t)RW * (2 * row0) : W.nrow + (size_t)RW * row0);
     if (mine) {
       const float* S = rows + (size_t)RW * (Fr ? 2 * q : q);
@@ -1395,12 +1408,17 @@ __device__ __forceinline__ bool flowRun(const FlowSweep& W, const SolverParams& 
       }
     }
   }
+  // each row's scalars on the whole quad: jacInv and friction coefficient, or jacInv, restitution and (below) the part of
+  // the impulse without velocities; most: the wave's most points of a slot
+  float jac[NV], coef[NV], part[NV];
+  spreadScalars<Fr>(s15, s16, s17, s18, jac, coef);
+  const int most = __any(nr > 2) ? (__any(nr > 3) ? 4 : 3) : (__any(nr > 1) ? 2 : 1);
   const bool dyn = deg > 0, moves = invMass != 0.0f;
   V3 v = v3(0.0f, 0.0f, 0.0f);
   if (G.valid && !dyn) v = ld3(W.svel + 8 * (size_t)x + 4 * (q & 1));  // a static body's constant velocity
   // two static bodies (a caller's island list): nothing orders the sweeps of this slot but its own impulses
   const bool fixed = (d.x | d.y) == 0;
-  float old0 = 0.0f, old1 = 0.0f, total = 0.0f, pimp = 0.0f;
+  float old0 = 0.0f, old1 = 0.0f, total = 0.0f;
   bool pending = G.valid, needBody = G.valid && dyn, needImp = mine;
   for (int spin = 0;; spin++) {
     int away = 0;  // updates this lane's body still has to see
@@ -1418,7 +1436,11 @@ __device__ __forceinline__ bool flowRun(const FlowSweep& W, const SolverParams& 
     }
     if (!Fr && spin == 0) {  // the part of the impulse without velocities, while the first polls are out
       const float positionalError = -s16 * SP.erp / SP.dt;
-      pimp = positionalError * s15;
+      const float pimp = positionalError * s15;
+      part[0] = quadBcast<0>(pimp);
+      part[1] = quadBcast<1>(pimp);
+      part[2] = quadBcast<2>(pimp);
+      part[3] = quadBcast<3>(pimp);
     }
     if (needBody) {
       needBody = flowVersion(w0) != want || flowVersion(w1) != want;
@@ -1441,15 +1463,15 @@ __device__ __forceinline__ bool flowRun(const FlowSweep& W, const SolverParams& 
     if (go) {
       float out0 = old0, out1 = old1;
       if (Fr) {
-        flowFrictionRound<0>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
-        flowFrictionRound<1>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
-        flowFrictionRound<2>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
-        flowFrictionRound<3>(q, nr, moves, D, U, total, s16, s15, old0, s18, s17, old1, v, out0, out1);
+        flowFrictionRound<0>(most, q, nr, moves, D, U, total, coef, jac, old0, old1, v, out0, out1);
+        flowFrictionRound<1>(most, q, nr, moves, D, U, total, coef, jac, old0, old1, v, out0, out1);
+        flowFrictionRound<2>(most, q, nr, moves, D, U, total, coef, jac, old0, old1, v, out0, out1);
+        flowFrictionRound<3>(most, q, nr, moves, D, U, total, coef, jac, old0, old1, v, out0, out1);
       } else {
-        flowNormalRound<0>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
-        flowNormalRound<1>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
-        flowNormalRound<2>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
-        flowNormalRound<3>(q, nr, moves, D, U, pimp, s17, s15, old0, v, out0);
+        flowNormalRound<0>(most, q, nr, moves, D, U, part, coef, jac, old0, v, out0);
+        flowNormalRound<1>(most, q, nr, moves, D, U, part, coef, jac, old0, v, out0);
+        flowNormalRound<2>(most, q, nr, moves, D, U, part, coef, jac, old0, v, out0);
+        flowNormalRound<3>(most, q, nr, moves, D, U, part, coef, jac, old0, v, out0);
       }
       if (dyn) {
         flow_t o0, o1;
@@ -3089,8 +3111,8 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   // All sweeps of an iteration (of the whole solve, where neither constraints nor a residual test stand between
   // iterations) are one launch; one launch per colour where blocks are swept apart, where a colour lies past the
   // bodies' 64-bit masks, or where a body flagged static has a mass (its slots share colours).  The 100k pile (243k
-  // slots, 24 colours, 20 iterations): 4.96 ms in 560 launches, 2.48 ms in one; 7.1k slots, 17 colours: 3.04 and
-  // 1.14 ms; 1.3k slots, 7 colours, 10 iterations: 0.55 and 0.23 ms.
+  // slots, 24 colours, 20 iterations): 4.96 ms in 560 launches, 2.34 ms in one; 7.1k slots, 17 colours: 3.04 and
+  // 1.03 ms; 1.3k slots, 7 colours, 10 iterations: 0.55 and 0.19 ms.
   const bool flow = !blocked && !manyColours && !c.oddBodies;
   if (!flow && headColors < c.ncolors) {
     std::vector<int> offs(c.colorOff.begin(), c.colorOff.end());
@@ -3204,7 +3226,8 @@ void solverSolve(Ctx& c, float dt, const std::vector<int>* explicitList) {
   int* flowErr = flow ? c.flowCtl.p + flowCtlWords - 1 : nullptr;
   // one launch of `sweeps` sweeps from sweep0 on; timed: with its own events
   auto flowSweep = [&](int sweep0, int sweeps, double* res, bool timed) {
-    // Waves beyond what the dependences keep busy only poll (their reads go past the L2).  Solve time by grid:
+    // Waves beyond what the dependences keep busy only poll (their reads go past the L2).  Solve time by grid (measured
+    // before the rows lost their branches, about 10% above now):
     // 243k slots (15.2k groups) 2.93 ms at 768 waves, 2.48 at 1536, 2.57 at 2048, 2.93 at 4096; 7.1k slots (460 groups)
     // 1.20 ms at 128, 1.14 at 192 and 256, 1.19 at 512; 1.3k slots (85 groups) 0.245 ms at 64, 0.225 at 128 to 256.
     const int groups = na / kFlowSlots + c.ncolors;  // at least the groups of a sweep
