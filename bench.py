@@ -248,7 +248,8 @@ def pmc_child(args):
     print(json.dumps({"rows": ks["rows"], "launches": ks["launches"]}))
 
 
-KERNEL_MATCH = {"friction": (r"kFriction\(", "%kFriction(%"), "normal": (r"kNormal\(", "%kNormal(%"),
+# a timed iteration launches its normal and its friction sweep one after the other with the same kernel
+KERNEL_MATCH = {"friction": (r"kFlowSweep\(", "%kFlowSweep(%"), "normal": (r"kFlowSweep\(", "%kFlowSweep(%"),
                 "friction_blocks": (r"kSweepBlocks<true>", "%kSweepBlocks<true>%"),
                 "normal_blocks": (r"kSweepBlocks<false>", "%kSweepBlocks<false>%")}
 
@@ -283,11 +284,15 @@ def traffic(args, kind, blocks, tail, warmup):
         cur = sqlite3.connect(dbs[0]).cursor()
         cols = [r[1] for r in cur.execute("pragma table_info(counters_collection)")]
         order = "dispatch_id" if "dispatch_id" in cols else "rowid"
-        # the sweep launches of the counted steps are the last `launches` dispatches of the kernel
-        q = (f"select avg(value), count(*) from (select value from counters_collection where counter_name = ? and "
-             f"kernel_name like ? order by {order} desc limit ?)")
-        kf, nkf = cur.execute(q, (counter, like, int(child["launches"]))).fetchone()
-        cp, ncp = cur.execute(q, (counter, "%kCopyProbe%", 1)).fetchone()
+        # the sweep launches of the counted steps are the last `launches` dispatches of the kernel, of the shared one
+        # every other (the last is a friction sweep)
+        q = f"select value from counters_collection where counter_name = ? and kernel_name like ? order by {order} desc limit ?"
+        skip, every = {"friction": (0, 2), "normal": (1, 2)}.get(kind, (0, 1))
+        values = [v for v, in cur.execute(q, (counter, like, every * int(child["launches"])))][skip::every]
+        nkf = len(values)
+        kf = sum(values) / max(nkf, 1)
+        copies = [v for v, in cur.execute(q, (counter, "%kCopyProbe%", 1))]
+        ncp, cp = len(copies), copies[0] if copies else 0
         log(f"[bench] counter pass {counter}: ordered by {order}, {nkf} sweep dispatches of the counted steps")
         if not nkf or not ncp or not cp or nkf != child["launches"]:
             return None, f"counter pass {counter}: no dispatches recorded"
@@ -339,8 +344,8 @@ def phase_roofline(tim, nsteps, st, args):
 
 def autotune(ctx, dt, steps=TUNE_STEPS):
     """Launch shaping of the sweeps (results are bit-identical for every choice): the block size of the
-    block-partitioned sweeps (0: one launch per colour) and, without blocks, the largest colour swept by the
-    single-workgroup tail launch.  Each candidate runs a few untimed warmup steps."""
+    block-partitioned sweeps (0: all sweeps of a solve in one launch) and the largest colour swept by the
+    single-workgroup tail launch, which only matters where a launch per colour is used.  Each candidate runs a few untimed warmup steps."""
     cands = TUNE_CANDIDATES
     ms = {}
     for blocks, tail in cands:
@@ -360,7 +365,7 @@ def autotune(ctx, dt, steps=TUNE_STEPS):
 
 
 def roofline(ks, args):
-    """Dominant kernel: the solver's colour sweeps.  The sampled launches (the sweeps of every fifth iteration on
+    """Dominant kernel: the solver's sweeps.  The sampled launches (the sweeps of every fifth iteration on
     a sampled step of the timed region) are each timed by their own start/stop events
     on the library stream (kernel execution only); achieved = algorithmic bytes per launch / average duration,
     with ROW_BYTES per row per sweep (80 B row + 4 B impulse + 2 x 48 B body velocity read and write)."""
@@ -371,7 +376,8 @@ def roofline(ks, args):
     avg_s = k["ms"] / k["launches"] / 1000.0
     bytes_per_launch = ROW_BYTES * k["rows"] / k["launches"]
     achieved = bytes_per_launch / avg_s / 1e9
-    kernel = {"normal": "kNormal (normal-row colour sweep)", "friction": "kFriction (friction-row colour sweep)",
+    kernel = {"normal": "kFlowSweep (a normal-row sweep over every colour)",
+              "friction": "kFlowSweep (a friction-row sweep over every colour)",
               "normal_blocks": "kSweepBlocks<false> (normal rows, block-partitioned sweep)",
               "friction_blocks": "kSweepBlocks<true> (friction rows, block-partitioned sweep)"}[name]
     others = {n: {"avg_launch_us": round(v["ms"] * 1e3 / v["launches"], 3), "launches_timed": v["launches"],
