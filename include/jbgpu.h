@@ -298,8 +298,8 @@ int jbgpu_solver_set_blocks(jbgpu_ctx* ctx, int32_t block_size);
  * block of its own, up to 1024 dynamic bodies): the workgroup colours the block's manifolds, applies the warm
  * start and runs every iteration with the block's velocities in LDS, so a solve is one launch.  The manifold
  * order (jbgpu_solver_get_order) is then block after block, colour after colour inside a block, reported as one
- * batch.  0 (the default) solves with one launch per colour batch.  Tolerance-driven solves (tolerance > 0)
- * always use the per-colour launches.  pipelined != 0: while a colour is swept, the rows of the next colour are
+ * batch.  0 (the default) solves the manifolds of all worlds together.  Tolerance-driven solves (tolerance > 0)
+ * always solve them together.  pipelined != 0: while a colour is swept, the rows of the next colour are
  * already being loaded (more registers per thread, fewer waves per SIMD). */
 int jbgpu_solver_set_world_blocks(jbgpu_ctx* ctx, int32_t bodies_per_block, int32_t threads, int32_t pipelined);
 /* Colouring of the manifolds into batches (no reference counterpart): Jones-Plassmann rounds with hashed
