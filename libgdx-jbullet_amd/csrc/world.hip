@@ -363,6 +363,7 @@ void uploadPairs(Ctx& c, int64_t n, const uint64_t* keys, const float* manifolds
   if (n) {
     c.host.send(c.stream, c.keys[c.cur].p, keys, n * sizeof(uint64_t));
     c.host.send(c.stream, c.man[c.cur].p, manifolds, (size_t)n * JBGPU_MANIFOLD_WORDS * sizeof(float));
+    JB_CHECK(hipStreamSynchronize(c.stream));  // the caller's arrays are free again, whichever way they went
   }
   c.npairs = n;
   c.npairsOld = 0;

@@ -40,7 +40,7 @@ class CopyPool {
 class HostCopy {
  public:
   ~HostCopy();
-  // queues dev[0, bytes) = host[0, bytes) on the stream; the host memory has been read when it returns
+  // queues dev[0, bytes) = host[0, bytes) on the stream; the host memory has to live until the stream gets there
   void send(hipStream_t s, void* dev, const void* host, size_t bytes);
   // host[0, bytes) = dev[0, bytes) after everything queued before; returns when the host memory holds it
   void fetch(hipStream_t s, void* host, const void* dev, size_t bytes);
