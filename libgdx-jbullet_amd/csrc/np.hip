@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kBinOrderThreads) void kBinOrder(int n, const int* 
   at[t] = 0;
   const int per = ((n + kWaves - 1) / kWaves + 63) / 64 * 64;
   const int first = w * per;
-  // the lanes of this round with this lane's key
+  // the lanes whose pairs have this lane's key
   auto same = [&](bool valid, int key) {
     unsigned long long m = __ballot(valid);
     for (int b = 0; b < 2 + kBinClassBits; b++) {
